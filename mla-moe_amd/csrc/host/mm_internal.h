@@ -20,6 +20,13 @@ typedef enum {
     K_MOE_BF16_S2L,
     K_MOE_BF16_S3,
     K_MOE_BF16_S3L,
+    K_BF16_ROWS,
+    K_BF16_GU_16,
+    K_BF16_GU_32,
+    K_BF16_GU_64,
+    K_BF16_DN_16,
+    K_BF16_DN_32,
+    K_BF16_DN_64,
     K_FILL,
     K_QUANT_W,
     K_I8_ROUTE,

@@ -509,7 +509,150 @@ static int launch_s2(mm_ctx *c, unsigned gx, unsigned gy, mm_gu_bf16_args *a) {
     return mm_launch(c, staged ? K_MOE_BF16_S2L : K_MOE_BF16_S2, gx, gy, 1, 256, staged ? xl : 0, a);
 }
 
-/* bf16 weights, GEMV stages (kernels/moe_bf16.hip), BF16_NT_MAX tokens per pass. */
+static int launch_router_logits(mm_ctx *c, mm_router_args *a);
+static int clear_counters(mm_ctx *c, int st);
+
+/* The grouped-GEMM form's workspace for T tokens (offsets into one region). */
+typedef struct {
+    size_t rows, inv, xs, xt, h, hs, y, ys, idx, wts, lg, bytes;
+} bf16_mm_plan;
+
+static bf16_mm_plan bf16_mm_layout(const mm_moe_config *g, size_t T, int logits) {
+    const size_t H = g->hidden_size, E = g->n_routed_experts, K = g->n_experts_per_tok;
+    const size_t I = g->moe_inter_size, S = (size_t)g->n_shared_experts * I, R = T * K;
+    mm_plan p = {0};
+    bf16_mm_plan w;
+    w.rows = plan_take(&p, E * T * 4);
+    w.inv = plan_take(&p, R * 4);
+    w.xs = plan_take(&p, 3 * R * H * 2);
+    w.xt = plan_take(&p, S ? 3 * T * H * 2 : 0);
+    w.h = plan_take(&p, 3 * R * I * 2);
+    w.hs = plan_take(&p, 3 * T * S * 2);
+    w.y = plan_take(&p, R * H * 4);
+    w.ys = plan_take(&p, S ? T * H * 4 : 0);
+    w.idx = plan_take(&p, R * 4);
+    w.wts = plan_take(&p, R * 4);
+    w.lg = plan_take(&p, logits ? 0 : T * E * 4);
+    w.bytes = p.off;
+    return w;
+}
+
+/* Weight matrices and activation tiles are read through 32-bit buffer offsets. */
+static int bf16_mm_ok(const mm_moe_config *g) {
+    const size_t H = g->hidden_size, I = g->moe_inter_size, S = (size_t)g->n_shared_experts * I;
+    return I * H < 0x7FFF0000u && S * H < 0x7FFF0000u;
+}
+
+/* One pass over T tokens: router logits, routing with per-expert row lists,
+ * the sorted planes of x, gate/up, down, combine. */
+static int bf16_mm_pass(mm_ctx *c, const mm_moe_layer *L, int T, const float *xn, float *out,
+                        const float *logits, int32_t *idx, float *wts, float *probs, int acc,
+                        const bf16_mm_plan *w, char *ws) {
+    const mm_moe_config *g = &c->moe;
+    const int H = g->hidden_size, E = g->n_routed_experts, K = g->n_experts_per_tok;
+    const int I = g->moe_inter_size, S = g->n_shared_experts * I, R = T * K;
+    int st;
+    if (!idx) idx = (int32_t *)(ws + w->idx);
+    if (!wts) wts = (float *)(ws + w->wts);
+    int32_t *rows = (int32_t *)(ws + w->rows), *inv = (int32_t *)(ws + w->inv);
+    if (!logits) {
+        mm_router_args la;
+        memset(&la, 0, sizeof(la));
+        la.x = xn;
+        la.wg = L->wg;
+        la.logits_out = (float *)(ws + w->lg);
+        la.T = T;
+        la.H = H;
+        la.E = E;
+        la.K = K;
+        if ((st = launch_router_logits(c, &la))) return st;
+        logits = la.logits_out;
+    }
+    mm_i8_route_args ra;
+    memset(&ra, 0, sizeof(ra));
+    ra.r.x = xn;
+    ra.r.logits_in = logits;
+    ra.r.bias = L->bias;
+    ra.r.probs = probs;
+    ra.r.topk_idx = idx;
+    ra.r.topk_w = wts;
+    ra.r.T = T;
+    ra.r.H = H;
+    ra.r.E = E;
+    ra.r.K = K;
+    ra.r.sigmoid = g->router_sigmoid;
+    ra.r.norm_topk = g->norm_topk;
+    ra.r.scale = g->routed_scaling;
+    ra.cnt = c->moe_cnt;
+    ra.rows = rows;
+    if (E > MM_EMAX_FAST)
+        st = route_wide(c, L, T, xn, logits, NULL, idx, wts, probs, &ra);
+    else
+        st = mm_launch(c, K_I8_ROUTE, (T + MM_I8_RT_TOKENS - 1) / MM_I8_RT_TOKENS, 1, 1,
+                       2 * 64 * MM_I8_RT_WAVES, 0, &ra);
+    if (st) return clear_counters(c, st);
+    mm_bf16_rows_args xa = {xn, c->moe_cnt, rows, inv, (uint16_t *)(ws + w->xs), (uint16_t *)(ws + w->xt),
+                            T, H, E, K, R};
+    if ((st = mm_launch(c, K_BF16_ROWS, (unsigned)(R + (S ? T : 0)), 1, 1, 256, 0, &xa)))
+        return clear_counters(c, st);
+    /* rows per tile by the mean rows of an expert (R routes over E): fewer
+     * rows leave LDS for a deeper weight ring, more read an expert's weights
+     * fewer times */
+    const size_t mean = ((size_t)R + E - 1) / E;
+    const int bm = mean <= 8 ? 0 : mean <= 24 ? 1 : 2;
+    static const mm_kernel_id kgu[3] = {K_BF16_GU_16, K_BF16_GU_32, K_BF16_GU_64};
+    static const mm_kernel_id kdn[3] = {K_BF16_DN_16, K_BF16_DN_32, K_BF16_DN_64};
+    static const size_t lds[3] = {MM_BF16_MM_LDS(16), MM_BF16_MM_LDS(32), MM_BF16_MM_LDS(64)};
+    mm_bf16_mm_args ga;
+    memset(&ga, 0, sizeof(ga));
+    ga.cnt = c->moe_cnt;
+    ga.nseg = S ? 2 : 1;
+    ga.T = T;
+    ga.E = E;
+    const size_t IH = (size_t)I * H;
+    ga.seg[0] = (mm_bf16_mm_seg){L->eg, L->eu, IH, xa.xs, (size_t)R * H, (uint16_t *)(ws + w->h),
+                                 (size_t)R * I, NULL, I, H};
+    ga.seg[1] = (mm_bf16_mm_seg){L->sg, L->su, 0, xa.xt, (size_t)T * H, (uint16_t *)(ws + w->hs),
+                                 (size_t)T * S, NULL, S, H};
+    if ((st = mm_launch(c, kgu[bm], MM_BF16_MM_GRID, 1, 1, MM_BF16_MM_THREADS, lds[bm], &ga))) return clear_counters(c, st);
+    ga.seg[0] = (mm_bf16_mm_seg){L->ed, NULL, IH, (uint16_t *)(ws + w->h), (size_t)R * I, NULL, 0,
+                                 (float *)(ws + w->y), H, I};
+    ga.seg[1] = (mm_bf16_mm_seg){L->sd, NULL, 0, (uint16_t *)(ws + w->hs), (size_t)T * S, NULL, 0,
+                                 (float *)(ws + w->ys), H, S};
+    if ((st = mm_launch(c, kdn[bm], MM_BF16_MM_GRID, 1, 1, MM_BF16_MM_THREADS, lds[bm], &ga))) return clear_counters(c, st);
+    mm_i8_combine_args ca = {(float *)(ws + w->y), (float *)(ws + w->ys), wts, out, c->moe_cnt, T, H, K, E,
+                             acc, S > 0, NULL, NULL, 0.0f, NULL, inv};
+    if ((st = mm_launch(c, K_I8_COMBINE, (unsigned)T, 2, 1, 256, 0, &ca))) return clear_counters(c, st);
+    return MM_OK;
+}
+
+/* bf16 weights as grouped GEMMs (kernels/moe_bf16_mm.hip), in passes of at
+ * most MM_BF16_MM_T_CHUNK tokens, or of as many as a fixed workspace holds
+ * (a token's results do not depend on the pass it is in).  *fits is 0, and
+ * nothing has run, when the fixed workspace cannot hold one token. */
+static int forward_bf16_mm(mm_ctx *c, const mm_moe_layer *L, int T, const float *xn, float *out,
+                           const float *logits, int32_t *idx, float *wts, float *probs, int acc,
+                           const mm_fixed_ws *fx, int *fits) {
+    const mm_moe_config *g = &c->moe;
+    const size_t H = g->hidden_size, E = g->n_routed_experts, K = g->n_experts_per_tok;
+    int tc = T < MM_BF16_MM_T_CHUNK ? T : MM_BF16_MM_T_CHUNK;
+    if (fx)
+        while (tc > 0 && bf16_mm_layout(g, tc, logits != NULL).bytes > fx->cap) tc -= (tc + 15) / 16;
+    *fits = tc > 0;
+    if (!*fits) return MM_OK;
+    const bf16_mm_plan w = bf16_mm_layout(g, tc, logits != NULL);
+    char *ws;
+    int st = take_ws(c, fx, w.bytes, &ws);
+    for (int t0 = 0; t0 < T && !st; t0 += tc)
+        st = bf16_mm_pass(c, L, T - t0 < tc ? T - t0 : tc, xn + (size_t)t0 * H, out + (size_t)t0 * H,
+                          logits ? logits + (size_t)t0 * E : NULL, idx ? idx + (size_t)t0 * K : NULL,
+                          wts ? wts + (size_t)t0 * K : NULL, probs ? probs + (size_t)t0 * E : NULL, acc, &w,
+                          ws);
+    return st;
+}
+
+/* bf16 weights: grouped GEMMs from MM_BF16_MM_MIN_T tokens on, else the GEMV
+ * stages (kernels/moe_bf16.hip), BF16_NT_MAX tokens per pass. */
 static int forward_bf16(mm_ctx *c, const mm_moe_layer *L, int T, const float *xn, float *out,
                         const float *logits, int32_t *idx, float *wts, float *probs, int acc,
                         const mm_fixed_ws *fx) {
@@ -518,6 +661,11 @@ static int forward_bf16(mm_ctx *c, const mm_moe_layer *L, int T, const float *xn
     const int I = g->moe_inter_size, S = g->n_shared_experts * I;
     const size_t hw = (size_t)K * I + S;
     const int wide = E > MM_EMAX_FAST;
+    if (T >= MM_BF16_MM_MIN_T && bf16_mm_ok(g)) {
+        int fits;
+        const int st = forward_bf16_mm(c, L, T, xn, out, logits, idx, wts, probs, acc, fx, &fits);
+        if (st || fits) return st;
+    }
     mm_plan p = {0};
     const size_t o_h = plan_take(&p, (size_t)BF16_NT_MAX * hw * sizeof(float));
     const size_t o_i = plan_take(&p, (size_t)T * K * sizeof(int32_t));
@@ -847,7 +995,7 @@ static int forward_int8(mm_ctx *c, const mm_moe_layer *L, int T, const float *xn
 
     mm_i8_combine_args ca = {y, ys, wts, out, tiled ? c->moe_cnt : NULL, T, (int)H, (int)K,
                              (int)E, acc, S > 0, c->norm_w, c->norm_xn, c->norm_eps,
-                             c->norm_w ? c->norm_xn_hl : NULL};
+                             c->norm_w ? c->norm_xn_hl : NULL, NULL};
     if (c->norm_w)   /* one block per token, the row's norm in the same pass */
         FAIL_ROUTED(mm_launch(c, K_I8_COMBINE_NORM, (unsigned)T, 1, 1, MM_I8_CN_THREADS, 0, &ca));
     else             /* two blocks per token: one round of loads per thread at H = 2048 */

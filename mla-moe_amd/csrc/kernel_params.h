@@ -80,6 +80,56 @@ typedef struct {
     int rows_per_block;
 } mm_down_bf16_args;
 
+/* bf16 MoE as grouped GEMMs (moe_bf16_mm.hip), from MM_BF16_MM_MIN_T tokens
+ * on: the GEMV streams an expert once per token that chose it, the GEMMs once
+ * per row tile but through six launches (DeepSeek-V2-Lite layer, 4 tokens: 98
+ * us by GEMV, 103 by GEMM; 5: 127 and 115; 8: 186 and 143; 64: 1430 and 248). */
+#ifndef MM_BF16_MM_MIN_T
+#define MM_BF16_MM_MIN_T 5
+#endif
+#define MM_BF16_MM_T_CHUNK 2048   /* rows of one pass (its workspace: ~180 KB per row) */
+#define MM_BF16_MM_GRID 256       /* persistent grid: one block per CU */
+#define MM_BF16_MM_THREADS 320    /* four multiplying waves and one loading activations */
+/* The load rings of 16-, 32- and 64-row tiles (dynamic LDS): NSW stages of KB
+ * values of K of 128 weight rows, NSA of the three planes of the rows */
+#ifndef MM_BF16_MM_KB
+#define MM_BF16_MM_KB(bm) ((bm) == 16 ? 128 : 64)
+#define MM_BF16_MM_NSW(bm) ((bm) == 16 ? 4 : (bm) == 32 ? 7 : 5)
+#define MM_BF16_MM_NSA(bm) ((bm) == 16 ? 2 : 3)
+#endif
+#define MM_BF16_MM_LDS(bm) \
+    ((128 * MM_BF16_MM_NSW(bm) + 3 * (bm) * MM_BF16_MM_NSA(bm)) * 2 * MM_BF16_MM_KB(bm))
+
+/* Routes sorted by expert: inv[route] = sorted position, xs = x's rows in
+ * that order as three bf16 planes [3][R][H] summing to the fp32 values, xt
+ * the tokens' rows likewise [3][T][H].  Grid: R (+ T with xt) blocks. */
+typedef struct {
+    const float *x;          /* [T, H] */
+    const int32_t *cnt;      /* [E * MM_CNT_STRIDE] rows per expert */
+    const int32_t *rows;     /* [E, T] route ids (t*K + r) per expert */
+    int32_t *inv;            /* [R] */
+    uint16_t *xs, *xt;
+    int T, H, E, K, R;
+} mm_bf16_rows_args;
+
+/* One grouped GEMM: segment 0 the routed experts over the sorted routes,
+ * segment 1 the shared expert over the tokens. */
+typedef struct {
+    const uint16_t *w0, *w1; /* gate and up [N, Kd] of expert 0, or down and NULL */
+    size_t wstride;          /* elements between experts */
+    const uint16_t *a;       /* activation planes [3][rows][Kd] */
+    size_t aplane;           /* elements per plane */
+    uint16_t *h;             /* gate/up out: planes [3][rows][N] */
+    size_t hplane;
+    float *y;                /* down out: [rows, N] */
+    int N, Kd;
+} mm_bf16_mm_seg;
+typedef struct {
+    mm_bf16_mm_seg seg[2];
+    const int32_t *cnt;      /* [E * MM_CNT_STRIDE] */
+    int nseg, T, E;
+} mm_bf16_mm_args;
+
 /* Synthetic data and format conversion utilities. */
 typedef struct {
     void *dst;
@@ -166,7 +216,7 @@ typedef struct {
     int32_t *cnt;            /* [E * MM_CNT_STRIDE] rows per expert (zero on entry), or 0 */
     int32_t *rows;           /* [E, T] route ids (t*K + r) per expert, or 0 (no lists) */
     const float *x;          /* [T, H] */
-    int8_t *qx;              /* [T, H] */
+    int8_t *qx;              /* [T, H], or 0: x is not quantised */
     float *sx;               /* [T] */
 } mm_i8_route_args;
 
@@ -203,7 +253,8 @@ typedef struct {
     int rows2, n2;
 } mm_i8_quant_rows_args;
 
-/* out[t] (=|+=) sum_r w[t,r] * y[t*K + r] + ys[t]; clears the E counters
+/* out[t] (=|+=) sum_r w[t,r] * y[t*K + r] + ys[t] (with yrow, route t*K + r's
+ * row of y is yrow[t*K + r]); clears the E counters
  * cnt[e * MM_CNT_STRIDE] when cnt is given (the tiled path's per-expert
  * counters, read by then). */
 typedef struct {
@@ -219,6 +270,7 @@ typedef struct {
     float *xn;
     float eps;
     uint16_t *xn_hl;         /* or 0: xn also as bf16 hi/lo planes [2, T, H] */
+    const int32_t *yrow;     /* [T * K] or 0 (mm_i8_combine only) */
 } mm_i8_combine_args;
 #define MM_I8_CN_THREADS 512      /* mm_i8_combine_norm: one block per token */
 #define MM_I8_CN_MAXH 4096

@@ -120,6 +120,11 @@ __device__ __forceinline__ void lds_dma16_buf(uint32_t voff, rsrc_t r, uint32_t 
     asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
                  : : "v"(voff), "s"(r), "{m0}"(__builtin_amdgcn_readfirstlane(dst)) : "memory");
 }
+/* The same for bytes read once (non-temporal). */
+__device__ __forceinline__ void lds_dma16_buf_nt(uint32_t voff, rsrc_t r, uint32_t dst) {
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen nt lds"
+                 : : "v"(voff), "s"(r), "{m0}"(__builtin_amdgcn_readfirstlane(dst)) : "memory");
+}
 
 /* LDS byte address of a __shared__ location. */
 __device__ __forceinline__ uint32_t lds_addr(const void *p) {

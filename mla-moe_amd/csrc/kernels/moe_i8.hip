@@ -227,7 +227,7 @@ __device__ __forceinline__ void i8_route(const mm_i8_route_args &a) {
     const int tok = blockIdx.x * RT_TOKENS + (router ? wave : wave - MM_I8_RT_WAVES);
     if (!router) {
         /* quantising wave: its x row in one round trip, nothing shared */
-        if (tok < T) quant_row_wave(a.x + (size_t)tok * r.H, r.H, a.qx + (size_t)tok * r.H, a.sx + tok);
+        if (a.qx && tok < T) quant_row_wave(a.x + (size_t)tok * r.H, r.H, a.qx + (size_t)tok * r.H, a.sx + tok);
         if (a.rows) {   /* the block's barriers of the row-list pass */
             __syncthreads();
             __syncthreads();
@@ -865,7 +865,8 @@ extern "C" __global__ __launch_bounds__(256) void mm_i8_combine(mm_i8_combine_ar
 #pragma unroll
         for (int r = 0; r < MM_KMAX; r++)
             if (r < a.K) {
-                y[r] = *(const f32x4 *)(a.y + ((size_t)t * a.K + r) * a.H + n);
+                const size_t rid = (size_t)t * a.K + r;
+                y[r] = *(const f32x4 *)(a.y + (a.yrow ? (size_t)a.yrow[rid] : rid) * a.H + n);
                 wr[r] = w[r];
             }
         if (a.has_shared) ys = *(const f32x4 *)(a.ys + (size_t)t * a.H + n);

@@ -1,0 +1,131 @@
+"""The bf16 MoE layer as grouped GEMMs (more than a few tokens) at the edges
+of its tiles: 16-, 32- and 64-row tiles with remainders, experts with no row
+and with every row, hidden sizes that are no multiple of the 64-wide K chunk,
+column counts that are none of a tile's, no shared expert, more than 256
+experts, several passes, and values that fp32 barely holds.
+
+Bar: the weights and activations enter the products exactly (three bf16 parts
+of every fp32 value), so only fp32 sums round: with n = H and I terms the
+error of a sum of random terms is about sqrt(n) / 2 units of 2^-24 of its
+norm, here below 2e-6 of the layer output's 2-norm (measured 3e-7)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import mlamoe
+from mlamoe import synth
+
+pytestmark = pytest.mark.gpu
+TOL = 2e-6
+
+
+def ref64(w, x, idx, wt, NS):
+    f = lambda a: synth.bf16_to_f32(a).astype(np.float64)  # noqa: E731
+    x = x.astype(np.float64)
+
+    def mlp(v, g, u, d):
+        a, b = v @ f(g).T, v @ f(u).T
+        return (a / (1 + np.exp(-a)) * b) @ f(d).T
+    out = mlp(x, w["sg"], w["su"], w["sd"]) if NS else np.zeros_like(x)
+    for e in np.unique(idx):
+        t, r = np.nonzero(idx == e)
+        out[t] += wt[t, r, None].astype(np.float64) * mlp(x[t], w["eg"][e], w["eu"][e], w["ed"][e])
+    return out
+
+
+def run(H, E, K, I, NS, T, hot=False, scale=1.0, seed=0, chunk=None):
+    w = synth.moe_layer(900 + seed, H, E, I, NS)
+    x = synth.activations(901 + seed, T, H) * np.float32(scale)
+    lg = synth.uniform_logits(902 + seed, T, E)
+    if hot:                       # every token takes expert 1; expert 0 gets none
+        lg[:, 1] += 9
+        lg[:, 0] -= 9
+    with mlamoe.Context(0) as ctx:
+        ctx.moe_init(H, E, NS, K, I)
+        ctx.moe_load_layer(0, w, mlamoe.MM_LOAD_BF16)
+        out, idx, wt, _ = ctx.moe_forward(0, x, logits=lg)
+        again, *_ = ctx.moe_forward(0, x, logits=lg)
+    assert np.array_equal(out, again)           # the counters were left clear
+    ref = ref64(w, x, idx, wt, NS)
+    err = np.linalg.norm(out - ref) / np.linalg.norm(ref)
+    print(f"H={H} E={E} K={K} I={I} NS={NS} T={T} hot={hot}: {err:.2e}", flush=True)
+    assert err < TOL
+    return out
+
+
+@pytest.mark.parametrize("T", [5, 6, 16, 17, 33, 64, 65, 131])
+@pytest.mark.parametrize("hot", [False, True])
+def test_row_tiles(T, hot):
+    run(256, 8, 2, 128, 2, T, hot, seed=T)
+
+
+@pytest.mark.parametrize("H,E,K,I,NS,T", [(264, 4, 2, 72, 1, 70), (72, 3, 1, 8, 0, 40), (1032, 6, 3, 136, 1, 9),
+                                          (256, 300, 8, 64, 1, 37), (128, 160, 4, 64, 3, 90), (64, 2, 2, 200, 2, 300)])
+def test_shapes(H, E, K, I, NS, T):
+    run(H, E, K, I, NS, T, seed=H + I)
+
+
+def test_passes_agree():
+    """2,100 tokens (two passes) against the same rows alone: a row's result
+    does not depend on the rows beside it."""
+    H, E, K, I, NS, T = 64, 4, 2, 64, 1, 2100
+    w, x = synth.moe_layer(950, H, E, I, NS), synth.activations(951, T, H)
+    lg = synth.uniform_logits(952, T, E)
+    with mlamoe.Context(0) as ctx:
+        ctx.moe_init(H, E, NS, K, I)
+        ctx.moe_load_layer(0, w, mlamoe.MM_LOAD_BF16)
+        out, *_ = ctx.moe_forward(0, x, logits=lg)
+        part, *_ = ctx.moe_forward(0, x[2040:2060], logits=lg[2040:2060])
+    assert np.array_equal(out[2040:2060], part)
+
+
+def test_fixed_workspace():
+    """The no-allocation entry point takes as many tokens per pass as its
+    scratch holds: the same bits as the growing workspace."""
+    H, E, K, I, NS, T = 1024, 8, 4, 512, 2, 700
+    w, x = synth.moe_layer(960, H, E, I, NS), synth.activations(961, T, H)
+    with mlamoe.Context(0) as ctx:
+        ctx.moe_init(H, E, NS, K, I)
+        ctx.moe_load_layer(0, w, mlamoe.MM_LOAD_BF16)
+        dx = ctx.to_device(x)
+        a, b = ctx.empty((T, H), np.float32), ctx.empty((T, H), np.float32)
+        mlamoe._check(mlamoe.lib().mm_moe_forward_noalloc_dev(ctx.h, 0, T, dx.ptr, a.ptr, None, None, None, None,
+                                                              C.c_uint(mlamoe.MM_FWD_BF16)))
+        assert ctx.workspace_bytes() == 0
+        ctx.moe_forward_dev(0, T, dx, b)
+        assert np.array_equal(a.download(), b.download())
+
+
+@pytest.mark.parametrize("inf", [False, True])
+def test_large_and_infinite_activations(inf):
+    """Activations near the largest fp32 value split without overflow; an
+    infinite one gives infinity, as fp32 arithmetic does (weights positive
+    where it meets them: infinity times zero is NaN in either)."""
+    H, E, K, I, NS, T = 64, 2, 1, 64, 0, 20
+    w = synth.moe_layer(970, H, E, I, NS)
+    one = np.uint16(0x3f80)
+    x = np.zeros((T, H), np.float32)
+    if inf:
+        for k in ("eg", "eu", "ed"):
+            w[k] = np.full_like(w[k], one)             # g = u = sum x, out = I silu(g) u
+        x[:, 0] = 2.0
+        x[3, 0] = np.inf
+        want = np.where(np.arange(T) == 3, np.inf, I * 4.0 / (1 + np.exp(-2.0)))
+    else:
+        for k in ("eg", "eu", "ed"):
+            w[k] = np.zeros_like(w[k])
+        w["eu"][:, 0, 0] = w["eg"][:, 0, 1] = one      # u[0] = x[0], g[0] = x[1]
+        w["ed"][:, :, 0] = one                         # out = h[0]
+        x[:, 0] = np.float32(8e36)
+        x[:, 1] = 40.0                                 # silu(40) = 40
+        want = np.full(T, 40.0 * np.float64(np.float32(8e36)))
+    lg = synth.uniform_logits(971, T, E)
+    with mlamoe.Context(0) as ctx:
+        ctx.moe_init(H, E, NS, K, I)
+        ctx.moe_load_layer(0, w, mlamoe.MM_LOAD_BF16)
+        out, idx, wt, _ = ctx.moe_forward(0, x, logits=lg)
+    want = np.broadcast_to((wt[:, 0] * want)[:, None], out.shape)
+    fin = np.isfinite(want)
+    assert np.allclose(out[fin], want[fin], rtol=1e-6, atol=0)
+    assert np.array_equal(out[~fin], want[~fin])
