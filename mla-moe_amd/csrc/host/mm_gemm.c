@@ -51,7 +51,8 @@ size_t mm_gemm_bf16_ws_bytes(int T, int n_in, int d_out, unsigned flags) {
 }
 
 static int gemm_bf16_rows(mm_ctx *c, float *y, const uint16_t *xh, const uint16_t *xl,
-                          const uint16_t *w, int d_out, int n_in, int kp, int T, int split, int acc);
+                          const uint16_t *w, int d_out, float *y1, const uint16_t *w1, int d1, int n_in,
+                          int kp, int T, int split, int acc);
 static int cvt_rows(mm_ctx *c, const float *x, int n_in, int T, int split, char *ws,
                     uint16_t **xh, uint16_t **xl, int *kp);
 
@@ -84,8 +85,11 @@ int mm_gemm_bf16_ws2(mm_ctx *c, float *y0, const uint16_t *w0, int d0, float *y1
     uint16_t *xh, *xl;
     int kp;
     if ((st = cvt_rows(c, x, n_in, T, split, ws, &xh, &xl, &kp))) return st;
-    if ((st = gemm_bf16_rows(c, y0, xh, xl, w0, d0, n_in, kp, T, split, acc))) return st;
-    return d1 ? gemm_bf16_rows(c, y1, xh, xl, w1, d1, n_in, kp, T, split, acc) : MM_OK;
+    if (acc && d1) {   /* the one-launch form accumulates into one matrix only */
+        if ((st = gemm_bf16_rows(c, y0, xh, xl, w0, d0, NULL, NULL, 0, n_in, kp, T, split, acc))) return st;
+        return gemm_bf16_rows(c, y1, xh, xl, w1, d1, NULL, NULL, 0, n_in, kp, T, split, acc);
+    }
+    return gemm_bf16_rows(c, y0, xh, xl, w0, d0, y1, w1, d1, n_in, kp, T, split, acc);
 }
 
 size_t mm_gemm_bf16_hl_ws_bytes(int T, int n_in, int d0, int d1) {
@@ -157,28 +161,37 @@ int mm_gemm_bf16_add_rmsnorm_hl(mm_ctx *c, float *x, const uint16_t *ahl, const 
     return mm_launch(c, K_REDUCE_RMSNORM, (unsigned)T, 1, 1, MM_RRN_THREADS, 0, &r);
 }
 
-/* y = x W^T on x already in bf16 rows of stride kp (xh, and xl with split) */
+/* y = x W^T (and y1 = x W1^T when d1 > 0) on x already in bf16 rows of
+ * stride kp (xh, and xl with split) */
 static int gemm_bf16_rows(mm_ctx *c, float *y, const uint16_t *xh, const uint16_t *xl,
-                          const uint16_t *w, int d_out, int n_in, int kp, int T, int split, int acc) {
+                          const uint16_t *w, int d_out, float *y1, const uint16_t *w1, int d1, int n_in,
+                          int kp, int T, int split, int acc) {
     /* block tile columns: the widest of 128, 64, 32 that still gives 192
      * tiles (most of the 256 CUs), else 32 -- the projections of this path
      * have too few 128 x 128 tiles to fill the machine (measured per width) */
-    const size_t nby = ((size_t)T + 127) / 128;
+    const size_t nby = ((size_t)T + MM_GB_BM - 1) / MM_GB_BM;
     int bn = 32;
     for (int cw = 128; cw >= 64; cw /= 2)
-        if (((size_t)d_out + cw - 1) / cw * nby >= 192) {
+        if ((((size_t)d_out + cw - 1) / cw + ((size_t)d1 + cw - 1) / cw) * nby >= 192) {
             bn = cw;
             break;
         }
-    const size_t nbx = ((size_t)d_out + bn - 1) / bn;
-    mm_gemm_bf16_args a = {xh, xl, w, y, T, d_out, n_in, kp, split, acc, bn};
-    /* LDS ring: 4 stages (3 for the hi/lo split) of A hi [, A lo] (16 KB
-     * each) and bn rows of B (128 B each); a 1-D grid of 8 XCD columns, each
-     * with every row block of its column blocks (the kernel maps blocks to
-     * tiles) */
-    const size_t stage = (size_t)(split ? 2 : 1) * 16384 + (size_t)bn * 128;
-    const size_t lds = (split ? 3 : 4) * stage;
-    return mm_launch(c, K_GEMM_BF16, (unsigned)(8 * ((nbx + 7) / 8) * nby), 1, 1, 256, lds, &a);
+    const size_t nb0 = ((size_t)d_out + bn - 1) / bn, nbx = nb0 + ((size_t)d1 + bn - 1) / bn;
+    /* the XCDs' rectangle of tiles: fewest rounds of an XCD's 32 CUs, then
+     * fewest operand rows read into an XCD's L2 (x rows count once per plane) */
+    size_t best = 0, blocks = 0;
+    int xr = 1;
+    for (int r = 1; r <= 8; r *= 2) {
+        const size_t pr = (nby + r - 1) / r, pc = (nbx + 8 / r - 1) / (8 / r);
+        const size_t cost = ((pr * pc + 31) / 32 << 32) + pr * MM_GB_BM * (split ? 2 : 1) + pc * bn;
+        if (r > 1 && cost >= best) continue;
+        best = cost;
+        xr = r;
+        blocks = 8 * pr * pc;
+    }
+    mm_gemm_bf16_args a = {xh, xl, w, y, T, d_out, n_in, kp, split, acc, bn, (int)nb0, d1 ? w1 : NULL, y1, d1, xr};
+    const size_t lds = (size_t)MM_GB_NS(split, bn) * MM_GB_STAGE(split, bn);
+    return mm_launch(c, K_GEMM_BF16, (unsigned)blocks, 1, 1, 512, lds, &a);
 }
 
 /* x as bf16 rows of a stride padded to 64 (zeros past n_in) into ws: hi,
@@ -202,7 +215,7 @@ int mm_gemm_bf16_ws(mm_ctx *c, float *y, const float *x, const uint16_t *w, int 
     uint16_t *xh, *xl;
     int kp, st;
     if ((st = cvt_rows(c, x, n_in, T, split, ws, &xh, &xl, &kp))) return st;
-    return gemm_bf16_rows(c, y, xh, xl, w, d_out, n_in, kp, T, split, acc);
+    return gemm_bf16_rows(c, y, xh, xl, w, d_out, NULL, NULL, 0, n_in, kp, T, split, acc);
 }
 
 unsigned mm_gemv_blocks(int rows) {

@@ -80,7 +80,7 @@ typedef struct {
     int rows_per_block;
 } mm_down_bf16_args;
 
-/* bf16 MoE as grouped GEMMs (moe_bf16_mm.hip), from MM_BF16_MM_MIN_T tokens
+/* bf16 MoE as grouped GEMMs (moe_bf16_mm.h), from MM_BF16_MM_MIN_T tokens
  * on: the GEMV streams an expert once per token that chose it, the GEMMs once
  * per row tile but through six launches (DeepSeek-V2-Lite layer, 4 tokens: 98
  * us by GEMV, 103 by GEMM; 5: 127 and 115; 8: 186 and 143; 64: 1430 and 248). */
@@ -456,7 +456,19 @@ typedef struct {
     int split;               /* 1: two MFMAs per product (x = hi + lo) */
     int accumulate;
     int bn;                  /* block tile columns: 128, 64 or 32 */
+    int nb0;                 /* column blocks of w */
+    /* an optional second matrix over the same x (never accumulated): column
+     * blocks from nb0 on are its (w1 [d_out1, n_in] -> y1 [T, d_out1]) */
+    const uint16_t *w1;
+    float *y1;
+    int d_out1;
+    int xr;                  /* the 8 XCDs as xr x 8 / xr rectangles of tiles: 1, 2, 4 or 8 */
 } mm_gemm_bf16_args;
+#define MM_GB_BM 128
+/* LDS ring of mm_gemm_bf16: bytes per stage (A planes of 128 rows, bn rows of
+ * B, 128 B each) and stages */
+#define MM_GB_STAGE(split, bn) (((split) ? 32768 : 16384) + (bn) * 128)
+#define MM_GB_NS(split, bn) ((split) ? ((bn) == 32 ? 4 : 3) : (bn) == 128 ? 4 : (bn) == 64 ? 6 : 7)
 
 /* Skinny-M GEMM (T <= MM_SKINNY_T rows of x): block (MM_SKINNY_BN output columns,
  * one K split); partials [nsplit, T, d_out] when nsplit > 1. */

@@ -11,17 +11,14 @@
  * relative) so the result tracks the fp32 reference; A then stages exactly
  * like B.
  *
- * Block tile 128 x 128, K step 64; four waves in a 2 x 2 grid, each a 64 x
- * 64 tile (16 MFMAs per 32 of K).  Both operands stage through an LDS ring
- * (4 stages, 3 for the split) by direct loads issued three (two) steps
- * ahead of the MFMAs.
+ * See mm_gemm_bf16 for the tile and the two kinds of waves.
  */
 #include "common.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
 
-#define GB_BM 128
+#define GB_BM MM_GB_BM
 #define GB_BK 64
 #define GB_COPY (128 * 128)             /* A of one stage: 128 rows x 128 B */
 
@@ -53,178 +50,262 @@ extern "C" __global__ __launch_bounds__(256) void mm_cvt_bf16(mm_cvt_bf16_args a
     if (a.split) *(u16x8 *)(a.xl + i8 * 8) = lo;
 }
 
-/* Stage layout: [A hi][A lo (split mode)][B], each 128 rows (A) or output
- * columns (B) x 64 K = 16 KB.  A load instruction moves 8 rows x 128 B
- * (whole cache lines; half-line accesses measured ~2.6x slower): lane l
- * carries row 8 i + l / 8 and stores at position p = l % 8 of that row's
- * 128 B the 16 B chunk q = p ^ s(row), s(R) = (R / 2) % 8.  The XOR swizzle
- * makes the operand reads below (16 rows, one chunk each) conflict-free. */
+/* Block tile 128 rows x BN columns (128, 64 or 32), K chunks of 64, both
+ * operands global -> LDS by direct loads into a ring of NS stages [A hi][A lo
+ * (split mode)][B].  Eight waves, two per SIMD: four multiply (a 2 x 2 grid,
+ * 64 x BN / 2 each), four only load, NS - 1 chunks ahead.  A multiplying
+ * wave's instruction stream then holds nothing but LDS reads and MFMAs, the
+ * reads of the next 32-wide K step (the next chunk's first included: the
+ * barrier comes before a chunk's last MFMAs) between the MFMAs of the
+ * current one.  With four waves doing both in turn, the loads' issue, the
+ * reads' round trip and the MFMAs of a chunk added up (split mode, 2,048
+ * rows: 2,048 x 2,048 49 us, 2,048 x 10,944 209, 10,944 x 2,048 270; now 32,
+ * 153 and 178: 1,030-1,200 TFLOP/s of MFMAs, what a library product of 8,192
+ * cubed reaches here; 512 truncated rows through the four projections 59 us
+ * -> 39).  Its parts alone, 2,048 x 10,944: the loads 108 us (48 KB per chunk
+ * and CU: 20 TB/s out of L2), the MFMAs 100, both 153: they share the LDS.
+ *
+ * GB_FLUSH: the accumulators are added to a second set every 512 values of
+ * K (2,048 values, truncated input: error against 64 bits 2.7e-7 -> 1.3e-7).
+ *
+ * A load instruction moves 8 rows x 128 B (whole cache lines; half-line
+ * accesses measured ~2.6x slower): lane l carries row 8 i + l / 8 and stores
+ * at position l % 8 of that row's 128 B the 16 B piece (l % 8) ^ s(row), s(R)
+ * = (R / 2) % 8.  The XOR swizzle makes the operand reads (16 rows, one piece
+ * each) conflict-free.  Rows past T and columns past d_out, and weight pieces
+ * past n_in, are out of the buffers' range: nothing is read, zeros staged. */
 __device__ __forceinline__ int gb_swz(int R) { return (R >> 1) & 7; }
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+#define GB_OOB 0xFFFFFFF0u
+#define GB_FLUSH 8                /* chunks summed in one accumulator (512 values of K) */
 
-template <bool HL, int GB_BN>
+template <bool HL, int BN>
 __device__ __forceinline__ void gemm_block(const mm_gemm_bf16_args &a, uint8_t *lds) {
-    constexpr int GB_NC = GB_BN / 32;             /* B fragments of 16 columns per wave */
-    constexpr int NA = HL ? 2 : 1;                /* A copies: hi (and lo) */
-    constexpr int BOFF = NA * GB_COPY;
-    constexpr int SB = BOFF + GB_BN * 128;        /* stage bytes */
-    constexpr int NS = HL ? 3 : 4;                /* stages */
-    constexpr int D = NS - 1;                     /* steps issued ahead */
-    constexpr int G = 4 * NA + GB_NC;             /* transfers per wave per step */
+    constexpr int NP = HL ? 2 : 1;                 /* A planes: hi (and lo) */
+    constexpr int BOFF = NP * GB_COPY;
+    constexpr int SB = MM_GB_STAGE(HL, BN);
+    constexpr int NS = MM_GB_NS(HL, BN);
+    constexpr int LPW = 4 * NP + BN / 32;          /* loads per loading wave per chunk */
+    static_assert(SB == BOFF + BN * 128 && LPW * (NS - 2) < 64, "ring");
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
     /* 1-D grid: blocks are dealt to the 8 XCDs round robin (block b -> XCD
-     * b % 8).  XCD x takes the column blocks x, x + 8, ... for every row
-     * block: its weight columns are fetched into its L2 once and reused by
-     * all row blocks, and the x rows (small) are shared by its tiles */
-    const int nbx = (a.d_out + GB_BN - 1) / GB_BN, nby = (a.T + GB_BM - 1) / GB_BM;
-    const int b = blockIdx.x, slot = b / 8;
-    const int cb = b % 8 + 8 * (slot / nby), rb = slot % nby;
-    if (cb >= nbx) return;
-    const int m0 = rb * GB_BM, n0 = cb * GB_BN;
+     * b % 8).  The XCDs split the tile grid into xr x 8 / xr rectangles, so
+     * that an XCD's L2 takes in 1 / xr of x and xr / 8 of the weights (the host
+     * chooses xr).  Column blocks from nb0 on are the second matrix's. */
+    const int nb1 = a.w1 ? (a.d_out1 + BN - 1) / BN : 0;
+    const int nbx = a.nb0 + nb1, nby = (a.T + GB_BM - 1) / GB_BM;
+    const int xcd = blockIdx.x % 8, loc = blockIdx.x / 8, xc = 8 / a.xr;
+    const int pr = (nby + a.xr - 1) / a.xr, pc = (nbx + xc - 1) / xc;
+    const int rb = xcd / xc * pr + loc % pr;
+    int cb = xcd % xc * pc + loc / pr;
+    if (rb >= nby || loc % pr >= pr || loc / pr >= pc || cb >= nbx) return;
+    const bool second = cb >= a.nb0;
+    if (second) cb -= a.nb0;
+    const uint16_t *w = second ? a.w1 : a.w;
+    const int d_out = second ? a.d_out1 : a.d_out;
+    const int m0 = rb * GB_BM, n0 = cb * BN;
     const int K = a.n_in, KB = a.kp / GB_BK;
+    const uint32_t lds0 = lds_addr(lds);
 
-    /* wave w issues A instructions 4 w .. 4 w + 3 (rows 32 w .. 32 w + 31)
-     * (hi, lo) and B instructions GB_NC w .. GB_NC w + GB_NC - 1; rows past
-     * T / columns past d_out read the last one (results discarded); B chunks
-     * past n_in re-read chunk 0 of the row (A is zero there) */
-    const uint16_t *ah_src[4], *al_src[4], *b_src[GB_NC];
-    int bq[GB_NC];
+    if (wave >= 4) {   /* a loading wave: a quarter of each plane and of the weights */
+        const int lw = wave - 4, mrows = min(a.T - m0, GB_BM), ncols = min(d_out - n0, BN);
+        rsrc_t rs[NP + 1];
 #pragma unroll
-    for (int h = 0; h < 4; h++) {
-        const int R = 8 * (4 * wave + h) + (lane >> 3);
-        const int kq = 8 * ((lane & 7) ^ gb_swz(R));      /* element offset in the step */
-        const int m = min(m0 + R, a.T - 1);
-        ah_src[h] = a.xh + (size_t)m * a.kp + kq;
-        al_src[h] = HL ? a.xl + (size_t)m * a.kp + kq : nullptr;
-    }
+        for (int q = 0; q < NP; q++)
+            rs[q] = raw_rsrc((q ? a.xl : a.xh) + (size_t)m0 * a.kp, (uint32_t)mrows * (uint32_t)a.kp * 2u);
+        rs[NP] = raw_rsrc(w + (size_t)n0 * K, (uint32_t)ncols * (uint32_t)K * 2u);
+        constexpr int WL = BN / 32;                /* weight loads per wave: 8 rows each */
+        uint32_t ao[4], wo[WL];
+        int wk[WL];                                /* first K value of the lane's weight piece */
 #pragma unroll
-    for (int h = 0; h < GB_NC; h++) {
-        const int R = 8 * (GB_NC * wave + h) + (lane >> 3);
-        const int n = min(n0 + R, a.d_out - 1);
-        b_src[h] = a.w + (size_t)n * K;
-        bq[h] = 8 * ((lane & 7) ^ gb_swz(R));
-    }
-    auto issue = [&](int kb, int st) {
-        uint8_t *s0 = lds + st * SB;
-#pragma unroll
-        for (int h = 0; h < 4; h++) {
-            const int i = 4 * wave + h;
-            lds_dma16(ah_src[h] + kb * GB_BK, s0 + i * 1024);
-            if (HL) lds_dma16(al_src[h] + kb * GB_BK, s0 + GB_COPY + i * 1024);
+        for (int u = 0; u < 4; u++) {
+            const int R = 8 * (4 * lw + u) + (lane >> 3), kq = 8 * ((lane & 7) ^ gb_swz(R));
+            ao[u] = R < mrows ? ((uint32_t)R * (uint32_t)a.kp + (uint32_t)kq) * 2u : GB_OOB;
         }
 #pragma unroll
-        for (int h = 0; h < GB_NC; h++) {
-            const int k = kb * GB_BK + bq[h];
-            lds_dma16(b_src[h] + (k < K ? k : 0), s0 + BOFF + (GB_NC * wave + h) * 1024);
+        for (int u = 0; u < WL; u++) {
+            const int R = 8 * (WL * lw + u) + (lane >> 3);
+            wk[u] = 8 * ((lane & 7) ^ gb_swz(R));
+            wo[u] = R < ncols ? ((uint32_t)R * (uint32_t)K + (uint32_t)wk[u]) * 2u : GB_OOB;
+        }
+        auto issue = [&](int kb, int st) {         /* past the last chunk: the last again */
+            const int k0 = min(kb, KB - 1) * GB_BK;
+            const uint32_t sb = lds0 + (uint32_t)(st * SB);
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+#pragma unroll
+                for (int q = 0; q < NP; q++)
+                    lds_dma16_buf(ao[u] != GB_OOB ? ao[u] + (uint32_t)(2 * k0) : GB_OOB, rs[q],
+                                  sb + (uint32_t)(q * GB_COPY + (4 * lw + u) * 1024));
+#pragma unroll
+            for (int u = 0; u < WL; u++)
+                lds_dma16_buf(wo[u] != GB_OOB && k0 + wk[u] < K ? wo[u] + (uint32_t)(2 * k0) : GB_OOB, rs[NP],
+                              sb + (uint32_t)(BOFF + (WL * lw + u) * 1024));
+        };
+#pragma unroll 1
+        for (int s = 0; s < NS - 1; s++) issue(s, s);
+        VMCNT_WAIT(LPW * (NS - 2));                /* chunk 0 */
+        __builtin_amdgcn_s_barrier();
+        int st = NS - 1;
+        for (int kb = 0; kb < KB; kb++) {          /* one barrier per chunk */
+            issue(kb + NS - 1, st);                /* the slot of chunk kb - 1 */
+            st = st + 1 == NS ? 0 : st + 1;
+            VMCNT_WAIT(LPW * (NS - 2));            /* chunk kb + 1 */
+            __builtin_amdgcn_s_barrier();
+        }
+        VMCNT_WAIT(0);
+        if (BN < 64) __builtin_amdgcn_s_barrier();   /* before the multiplying waves' exchange */
+        return;
+    }
+
+    /* v_mfma_f32_32x32x16_bf16: operand lane l holds row (column) l % 32, K
+     * values 8 (l / 32) .. + 7 of a 16-wide step.  Row tile t (column tile j),
+     * step s: row 32 t + l % 32, piece 2 s + l / 32.  BN = 32: the waves of a
+     * row share its one column tile and split K's steps between them. */
+    constexpr int WT = BN >= 64 ? BN / 64 : 1;     /* 32-column tiles per wave */
+    constexpr int KH = BN >= 64 ? 1 : 2;           /* waves splitting a chunk's K */
+    constexpr int KS = 4 / KH;                     /* 16-wide steps per wave per chunk */
+    typedef const __attribute__((address_space(3))) i32x4 *lds_cp;
+    const int wm = wave >> 1, wn = wave & 1, c32 = lane & 31, hi = lane >> 5;
+    uint32_t rd[KS];
+#pragma unroll
+    for (int s = 0; s < KS; s++) rd[s] = c32 * 128 + 16 * ((2 * (KS * (KH > 1 ? wn : 0) + s) + hi) ^ gb_swz(c32));
+    const int cw = KH > 1 ? 0 : wn * (BN / 2);     /* the wave's first column */
+    i32x4 x[2][2][NP], wv[2][WT];
+    auto read = [&](int st, int s) {
+        const uint32_t sa = lds0 + (uint32_t)(st * SB) + rd[s] + wm * 64 * 128;
+        const uint32_t sw = lds0 + (uint32_t)(st * SB) + BOFF + rd[s] + cw * 128;
+#pragma unroll
+        for (int j = 0; j < WT; j++) wv[s & 1][j] = *(lds_cp)(sw + j * 4096);
+#pragma unroll
+        for (int q = 0; q < NP; q++)
+#pragma unroll
+            for (int t = 0; t < 2; t++) x[s & 1][t][q] = *(lds_cp)(sa + q * GB_COPY + t * 4096);
+    };
+    f32x16 acc[2][WT], sum[2][WT];
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int j = 0; j < WT; j++) acc[t][j] = sum[t][j] = (f32x16){};
+    auto mfma = [&](int s) {
+#pragma unroll
+        for (int q = 0; q < NP; q++)
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int j = 0; j < WT; j++)
+                    acc[t][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, wv[s & 1][j]),
+                                                                        __builtin_bit_cast(bf16x8, x[s & 1][t][q]),
+                                                                        acc[t][j], 0, 0, 0);
+        /* the reads between the MFMAs */
+        constexpr int RD = 2 * NP + WT, MF = 2 * NP * WT, PER = MF / RD > 0 ? MF / RD : 1;
+#pragma unroll
+        for (int i = 0; i < RD; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, PER, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
     };
-    /* operand read of lane (c = l % 16, g = l / 16) for fragment row block r
-     * and K half kh: row 16 r + c, chunk q = 4 kh + g, at (16 r + c) * 128 +
-     * 16 (q ^ s(c)); the r part is a compile-time offset */
-    const int c16 = lane & 15, g4 = lane >> 4;
-    const uint32_t rd0 = c16 * 128 + 16 * ((0 + g4) ^ gb_swz(c16));
-    const uint32_t rd1 = c16 * 128 + 16 * ((4 + g4) ^ gb_swz(c16));
-
-    f32x4 acc[4][GB_NC];
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    read(0, 0);
+    int st = 0;
+    for (int kb = 0; kb < KB; kb++) {
 #pragma unroll
-    for (int r = 0; r < 4; r++)
-#pragma unroll
-        for (int c = 0; c < GB_NC; c++) acc[r][c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-
-    /* every step issues one group (steps past the end re-load the last, so
-     * that the wait counts are static) */
-#pragma unroll
-    for (int s = 0; s < D; s++) issue(min(s, KB - 1), s);
-    __builtin_amdgcn_sched_barrier(0);
-    auto step = [&](int kb, int j) {   /* j = kb % NS */
-        VMCNT_WAIT(G * (D - 1));       /* this wave's step-kb group has landed */
-        __builtin_amdgcn_s_barrier();  /* ... every wave's, and stage kb-1 is free */
-        __builtin_amdgcn_sched_barrier(0);
-        issue(min(kb + D, KB - 1), (j + D) % NS);
-        __builtin_amdgcn_sched_barrier(0);
-        /* this wave's A rows 64 wm .. and B columns GB_BN / 2 * wn .. */
-        const uint32_t st0 = lds_addr(lds + j * SB);
-#pragma unroll
-        for (int kh = 0; kh < 2; kh++) {
-            const uint32_t sa = st0 + (kh ? rd1 : rd0) + wm * 64 * 128;
-            const uint32_t sb = st0 + BOFF + (kh ? rd1 : rd0) + wn * (GB_BN / 2) * 128;
-            i32x4 ah[4], al[4], bw[4];
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                ah[r] = ds_read16(sa, r * 2048);
-                if (HL) al[r] = ds_read16(sa, GB_COPY + r * 2048);
+        for (int s = 0; s < KS; s++) {
+            if (s + 1 < KS) {
+                read(st, s + 1);
+            } else {
+                /* this chunk's reads are done, so its slot may be refilled
+                 * after the barrier, which also shows every loading wave's
+                 * part of the next chunk */
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                st = st + 1 == NS ? 0 : st + 1;
+                read(st, 0);
             }
+            mfma(s);
+        }
+        if (kb % GB_FLUSH == GB_FLUSH - 1) {
 #pragma unroll
-            for (int c = 0; c < GB_NC; c++) bw[c] = ds_read16(sb, c * 2048);
-            if (HL)
-                asm volatile("s_waitcnt lgkmcnt(0)"
-                             : "+v"(ah[0]), "+v"(ah[1]), "+v"(ah[2]), "+v"(ah[3]), "+v"(al[0]), "+v"(al[1]),
-                               "+v"(al[2]), "+v"(al[3]), "+v"(bw[0]), "+v"(bw[1]), "+v"(bw[2]), "+v"(bw[3]));
-            else
-                asm volatile("s_waitcnt lgkmcnt(0)"
-                             : "+v"(ah[0]), "+v"(ah[1]), "+v"(ah[2]), "+v"(ah[3]), "+v"(bw[0]), "+v"(bw[1]),
-                               "+v"(bw[2]), "+v"(bw[3]));
+            for (int t = 0; t < 2; t++)
 #pragma unroll
-            for (int r = 0; r < 4; r++)
-#pragma unroll
-                for (int c = 0; c < GB_NC; c++) {
-                    const bf16x8 bb = __builtin_bit_cast(bf16x8, bw[c]);
-                    acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ah[r]), bb,
-                                                                        acc[r][c], 0, 0, 0);
-                    if (HL)
-                        acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, al[r]), bb,
-                                                                            acc[r][c], 0, 0, 0);
+                for (int j = 0; j < WT; j++) {
+                    sum[t][j] += acc[t][j];
+                    acc[t][j] = (f32x16){};
                 }
         }
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    int k0 = 0;
-    for (; k0 + NS <= KB; k0 += NS) {
-#pragma unroll
-        for (int j = 0; j < NS; j++) step(k0 + j, j);
     }
 #pragma unroll
-    for (int j = 0; j < NS - 1; j++)
-        if (k0 + j < KB) step(k0 + j, j);
-    VMCNT_WAIT(0);
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int j = 0; j < WT; j++) sum[t][j] += acc[t][j];
+    if (KH > 1) {
+        /* the odd wave's sums to the even one through the ring's LDS: free
+         * after a barrier (every load landed, every read done) */
+        typedef __attribute__((address_space(3))) float lds_f;
+        lds_f *red = (lds_f *)(lds0 + (uint32_t)(wm * 2 * 16 * MM_WAVE * 4 + lane * 4));
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (wn == 1) {
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) red[(16 * t + i) * MM_WAVE] = sum[t][0][i];
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (wn == 1) return;
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) sum[t][0][i] += red[(16 * t + i) * MM_WAVE];
+    }
 
-    /* lane holds D[4 (l / 16) + i][l % 16] of each 16 x 16 tile.  With
-     * accumulate, a row block's old outputs are all loaded (clamped
-     * addresses, unconditionally) before any is added: a load under the
-     * row / column conditions would be a branch of its own, each waited
-     * for before the next is issued. */
+    /* lane l holds row l % 32 and, in registers 4 g + i, columns 8 g + 4 (l /
+     * 32) + i of each 32 x 32 tile (the weights are the first operand).  With
+     * accumulate, a row tile's old outputs are all loaded (clamped addresses,
+     * unconditionally) before any is added. */
+    float *y = second ? a.y1 : a.y;
+    const bool acc_old = a.accumulate && !second;
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-        float prev[GB_NC][4];
-        if (a.accumulate) {   /* uniform */
+    for (int t = 0; t < 2; t++) {
+        const int m = m0 + 64 * wm + 32 * t + c32;
+        float *row = y + (size_t)min(m, a.T - 1) * d_out;
+        if (acc_old) {   /* uniform */
+            f32x16 prev[WT];
 #pragma unroll
-            for (int c = 0; c < GB_NC; c++)
+            for (int j = 0; j < WT; j++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int n = min(n0 + (GB_BN / 2) * wn + 16 * c + (lane & 15), a.d_out - 1);
-                    const int m = min(m0 + 64 * wm + 16 * r + 4 * (lane >> 4) + i, a.T - 1);
-                    prev[c][i] = a.y[(size_t)m * a.d_out + n];
+                for (int i = 0; i < 16; i++)
+                    prev[j][i] = row[min(n0 + cw + 32 * j + 8 * (i >> 2) + 4 * hi + (i & 3), d_out - 1)];
+#pragma unroll
+            for (int j = 0; j < WT; j++) sum[t][j] = prev[j] + sum[t][j];
+        }
+#pragma unroll
+        for (int j = 0; j < WT; j++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const int n = n0 + cw + 32 * j + 8 * g + 4 * hi;
+                if (m >= a.T || n >= d_out) continue;
+                if (n + 3 < d_out) {
+                    *(f32x4_a4 *)(row + n) = (f32x4){sum[t][j][4 * g], sum[t][j][4 * g + 1], sum[t][j][4 * g + 2],
+                                                     sum[t][j][4 * g + 3]};
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 3; i++)
+                        if (n + i < d_out) row[n + i] = sum[t][j][4 * g + i];
                 }
-        }
-#pragma unroll
-        for (int c = 0; c < GB_NC; c++) {
-            const int n = n0 + (GB_BN / 2) * wn + 16 * c + (lane & 15);
-            if (n >= a.d_out) continue;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int m = m0 + 64 * wm + 16 * r + 4 * (lane >> 4) + i;
-                if (m >= a.T) continue;
-                a.y[(size_t)m * a.d_out + n] = a.accumulate ? prev[c][i] + acc[r][c][i] : acc[r][c][i];
             }
-        }
     }
 }
 
-/* 1-D grid of 8 * ceil(ceil(d_out / 128) / 8) * ceil(T / 128) blocks, 256
- * threads, dynamic LDS: 4 stages x 32 KB (truncated x) or
- * 3 x 48 KB (hi/lo x). */
-extern "C" __global__ __launch_bounds__(256) void mm_gemm_bf16(mm_gemm_bf16_args a) {
+/* 1-D grid of 8 * ceil(row blocks / xr) * ceil(column blocks / (8 / xr))
+ * blocks, 512 threads, dynamic LDS: MM_GB_NS stages of MM_GB_STAGE bytes. */
+extern "C" __global__ __launch_bounds__(512, 1) void mm_gemm_bf16(mm_gemm_bf16_args a) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t glds[];
     if (a.split) {
         if (a.bn == 128) gemm_block<true, 128>(a, glds);
