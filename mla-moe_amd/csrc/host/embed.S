@@ -11,13 +11,6 @@ mm_co_moe_bf16:
     .incbin "moe_bf16.hsaco"
 
     .balign 4096
-    .globl mm_co_moe_bf16_mm
-    .hidden mm_co_moe_bf16_mm
-    .type mm_co_moe_bf16_mm, @object
-mm_co_moe_bf16_mm:
-    .incbin "moe_bf16_mm.hsaco"
-
-    .balign 4096
     .globl mm_co_util
     .hidden mm_co_util
     .type mm_co_util, @object

@@ -15,7 +15,6 @@
 
 /* ---- embedded code objects (embed.S) ------------------------------------ */
 extern const unsigned char mm_co_moe_bf16[];
-extern const unsigned char mm_co_moe_bf16_mm[];
 extern const unsigned char mm_co_util[];
 extern const unsigned char mm_co_moe_i8[];
 extern const unsigned char mm_co_mla[];
@@ -24,10 +23,9 @@ extern const unsigned char mm_co_gemm_i8[];
 extern const unsigned char mm_co_lm_head[];
 extern const unsigned char mm_co_gemv[];
 
-enum { MOD_MOE_BF16, MOD_MOE_BF16_MM, MOD_UTIL, MOD_MOE_I8, MOD_MLA, MOD_GEMM_BF16, MOD_GEMM_I8, MOD_LM_HEAD,
+enum { MOD_MOE_BF16, MOD_UTIL, MOD_MOE_I8, MOD_MLA, MOD_GEMM_BF16, MOD_GEMM_I8, MOD_LM_HEAD,
        MOD_GEMV, MOD_COUNT };
-static const unsigned char *const mod_blob[MOD_COUNT] = {mm_co_moe_bf16, mm_co_moe_bf16_mm,
-                                                          mm_co_util,
+static const unsigned char *const mod_blob[MOD_COUNT] = {mm_co_moe_bf16, mm_co_util,
                                                           mm_co_moe_i8, mm_co_mla,
                                                           mm_co_gemm_bf16, mm_co_gemm_i8,
                                                           mm_co_lm_head, mm_co_gemv};
@@ -45,13 +43,13 @@ static const struct {
     [K_MOE_BF16_S2L] = {"mm_moe_bf16_stage2_lds", MOD_MOE_BF16},
     [K_MOE_BF16_S3] = {"mm_moe_bf16_stage3", MOD_MOE_BF16},
     [K_MOE_BF16_S3L] = {"mm_moe_bf16_stage3_lds", MOD_MOE_BF16},
-    [K_BF16_ROWS] = {"mm_bf16_rows", MOD_MOE_BF16_MM},
-    [K_BF16_GU_16] = {"mm_bf16_gu_16", MOD_MOE_BF16_MM},
-    [K_BF16_GU_32] = {"mm_bf16_gu_32", MOD_MOE_BF16_MM},
-    [K_BF16_GU_64] = {"mm_bf16_gu_64", MOD_MOE_BF16_MM},
-    [K_BF16_DN_16] = {"mm_bf16_dn_16", MOD_MOE_BF16_MM},
-    [K_BF16_DN_32] = {"mm_bf16_dn_32", MOD_MOE_BF16_MM},
-    [K_BF16_DN_64] = {"mm_bf16_dn_64", MOD_MOE_BF16_MM},
+    [K_BF16_ROWS] = {"mm_bf16_rows", MOD_MOE_BF16},
+    [K_BF16_GU_16] = {"mm_bf16_gu_16", MOD_MOE_BF16},
+    [K_BF16_GU_32] = {"mm_bf16_gu_32", MOD_MOE_BF16},
+    [K_BF16_GU_64] = {"mm_bf16_gu_64", MOD_MOE_BF16},
+    [K_BF16_DN_16] = {"mm_bf16_dn_16", MOD_MOE_BF16},
+    [K_BF16_DN_32] = {"mm_bf16_dn_32", MOD_MOE_BF16},
+    [K_BF16_DN_64] = {"mm_bf16_dn_64", MOD_MOE_BF16},
     [K_FILL] = {"mm_fill", MOD_UTIL},
     [K_QUANT_W] = {"mm_quant_weight", MOD_UTIL},
     [K_I8_ROUTE] = {"mm_i8_route", MOD_MOE_I8},

@@ -626,7 +626,7 @@ static int bf16_mm_pass(mm_ctx *c, const mm_moe_layer *L, int T, const float *xn
     return MM_OK;
 }
 
-/* bf16 weights as grouped GEMMs (kernels/moe_bf16_mm.hip), in passes of at
+/* bf16 weights as grouped GEMMs (kernels/moe_bf16_mm.h), in passes of at
  * most MM_BF16_MM_T_CHUNK tokens, or of as many as a fixed workspace holds
  * (a token's results do not depend on the pass it is in).  *fits is 0, and
  * nothing has run, when the fixed workspace cannot hold one token. */

@@ -20,6 +20,7 @@
  * (w_r * silu(g) * u) so the combine of run.c:151-160 becomes a single dot
  * product over the concatenated hidden rows.
  */
+#include "moe_bf16_mm.h"
 #include "router.h"
 
 #define GU_THREADS 256

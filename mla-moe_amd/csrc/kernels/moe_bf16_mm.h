@@ -1,7 +1,8 @@
-/* moe_bf16_mm.hip -- MoE expert FFN with bf16 weights and fp32 activations
+/* moe_bf16_mm.h -- MoE expert FFN with bf16 weights and fp32 activations
  * for more than a few tokens: grouped GEMMs on v_mfma_f32_16x16x32_bf16.
  *
- * The GEMV stages (moe_bf16.hip) read a token's experts once per token; here
+ * The GEMV stages (moe_bf16.hip, whose module
+ * these kernels share) read a token's experts once per token; here
  * every touched expert's weights are read once per BM rows that chose it.
  * fp32 activations travel as three bf16 planes whose sum is exactly the fp32
  * value (split3: 8 + 8 + 8 significant bits), so every product is exact and
@@ -24,6 +25,7 @@
  * us (4.9 TB/s); with more rows per expert LDS reads and MFMAs share the time
  * (272 and 145 us at 515 tokens).
  */
+#pragma once
 #include "common.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -123,28 +125,28 @@ extern "C" __global__ __launch_bounds__(256) void mm_bf16_rows(mm_bf16_rows_args
  * step of the next chunk included: the wait for that chunk and the block's
  * barrier come before a chunk's last MFMAs.
  *
- * The sums of the hi planes move to a second set of registers every FLUSH
+ * The sums of the hi planes move to a second set of registers every GRP_FLUSH
  * values of K, those of the small planes have their own: one chain of K =
  * 2048 rounds to twice the error of the GEMV's 64 short chains. */
-#define NB 128                    /* weight rows per tile */
-#define OOB 0xFFFFFFF0u           /* past every buffer range */
-#define FLUSH 256
-#define MMW 4                     /* multiplying waves */
+#define GRP_NB 128                /* weight rows per tile */
+#define GRP_OOB 0xFFFFFFF0u           /* past every buffer range */
+#define GRP_FLUSH 256
+#define GRP_MMW 4                     /* multiplying waves */
 
 template <int BM> struct shape {
     static constexpr int KB = MM_BF16_MM_KB(BM);
     static constexpr int ROWB = 2 * KB;                /* LDS bytes per row */
     static constexpr int RPI = 1024 / ROWB;            /* rows per load instruction */
-    static constexpr int W_LPW = NB / RPI / MMW;       /* weight loads per wave per chunk */
+    static constexpr int W_LPW = GRP_NB / RPI / GRP_MMW;       /* weight loads per wave per chunk */
     static constexpr int A_INS = 3 * BM / RPI;         /* plane loads per chunk */
-    static constexpr int W_BYTES = NB * ROWB, A_BYTES = 3 * BM * ROWB;
+    static constexpr int W_BYTES = GRP_NB * ROWB, A_BYTES = 3 * BM * ROWB;
     static constexpr int NSW = MM_BF16_MM_NSW(BM), NSA = MM_BF16_MM_NSA(BM);
     static constexpr int WN = BM == 64 ? 2 : 4;        /* waves over the weight rows */
     static constexpr int TT = BM == 64 ? 2 : BM / 16;  /* 16-row tiles per wave */
-    static constexpr int WT = NB / 16 / WN;            /* 16-column weight tiles per wave */
+    static constexpr int WT = GRP_NB / 16 / WN;            /* 16-column weight tiles per wave */
     static constexpr int KS = KB / 32;                 /* MFMA steps per chunk */
     static_assert(NSW * W_BYTES + NSA * A_BYTES == MM_BF16_MM_LDS(BM), "ring sizes known to the host");
-    static_assert(W_LPW * (NSW - 2) < 64 && A_INS * (NSA - 2) < 64 && KS % 2 == 0 && FLUSH % KB == 0, "");
+    static_assert(W_LPW * (NSW - 2) < 64 && A_INS * (NSA - 2) < 64 && KS % 2 == 0 && GRP_FLUSH % KB == 0, "");
     static __device__ int swz(int r) { return KB == 64 ? (r >> 1) & 7 : r & 15; }
 };
 
@@ -163,7 +165,7 @@ struct grp_tile {
 
 template <int BM, bool GU>
 __device__ __forceinline__ grp_tile grp_decode(const mm_bf16_mm_args &a, const grp_shared &sh, int n0, int t) {
-    constexpr int CPT = GU ? NB / 2 : NB;
+    constexpr int CPT = GU ? GRP_NB / 2 : GRP_NB;
     grp_tile id;
     if (t < n0) {
         const int nslab = (a.seg[0].N + CPT - 1) / CPT;
@@ -200,7 +202,7 @@ __device__ __forceinline__ grp_tile grp_decode(const mm_bf16_mm_args &a, const g
 template <int BM, bool GU>
 __device__ __forceinline__ void grp_run(const mm_bf16_mm_args &a) {
     using sp = shape<BM>;
-    constexpr int CPT = GU ? NB / 2 : NB;              /* output columns per tile */
+    constexpr int CPT = GU ? GRP_NB / 2 : GRP_NB;              /* output columns per tile */
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     __shared__ grp_shared sh;
     const int tid = threadIdx.x, lane = tid & (MM_WAVE - 1);
@@ -270,7 +272,7 @@ __device__ __forceinline__ void grp_run(const mm_bf16_mm_args &a) {
         return true;
     };
 
-    if (wave == MMW) {   /* the planes' wave */
+    if (wave == GRP_MMW) {   /* the planes' wave */
         rsrc_t ar[3];
         constexpr int AP = sp::A_INS / 3;              /* loads per plane */
         uint32_t ao[AP];
@@ -286,7 +288,7 @@ __device__ __forceinline__ void grp_run(const mm_bf16_mm_args &a) {
 #pragma unroll
             for (int u = 0; u < AP; u++) {
                 const int R = RPI * u + lane / LPR;
-                ao[u] = R < rows ? ((uint32_t)R * (uint32_t)kd + (uint32_t)piece(R)) * 2u : OOB;
+                ao[u] = R < rows ? ((uint32_t)R * (uint32_t)kd + (uint32_t)piece(R)) * 2u : GRP_OOB;
             }
         };
         auto issue = [&](int slot) {
@@ -294,7 +296,7 @@ __device__ __forceinline__ void grp_run(const mm_bf16_mm_args &a) {
             const int k0 = ic * KB;
 #pragma unroll
             for (int u = 0; u < AP; u++) {
-                const uint32_t o = ao[u] != OOB && k0 + piece(RPI * u + lane / LPR) < kd ? ao[u] + (uint32_t)(2 * k0) : OOB;
+                const uint32_t o = ao[u] != GRP_OOB && k0 + piece(RPI * u + lane / LPR) < kd ? ao[u] + (uint32_t)(2 * k0) : GRP_OOB;
 #pragma unroll
                 for (int q = 0; q < 3; q++) lds_dma16_buf(o, ar[q], sb + (uint32_t)((q * AP + u) * 1024));
             }
@@ -322,7 +324,7 @@ __device__ __forceinline__ void grp_run(const mm_bf16_mm_args &a) {
     rsrc_t wr[GU ? 2 : 1];
     uint32_t wo[sp::W_LPW];
     auto wload_row = [&](int u) { return RPI * (sp::W_LPW * wave + u) + lane / LPR; };
-    auto wup = [&](int u) { return GU && RPI * (sp::W_LPW * wave + u) >= NB / 2; };   /* uniform */
+    auto wup = [&](int u) { return GU && RPI * (sp::W_LPW * wave + u) >= GRP_NB / 2; };   /* uniform */
     auto set_issue = [&](const grp_tile &id) {
         const mm_bf16_mm_seg &g = a.seg[id.si];
         kd = g.Kd;
@@ -332,7 +334,7 @@ __device__ __forceinline__ void grp_run(const mm_bf16_mm_args &a) {
 #pragma unroll
         for (int u = 0; u < sp::W_LPW; u++) {
             const int R = wload_row(u), col = id.slab * CPT + (GU ? R & 63 : R);
-            wo[u] = col < g.N ? ((uint32_t)col * (uint32_t)kd + (uint32_t)piece(R)) * 2u : OOB;
+            wo[u] = col < g.N ? ((uint32_t)col * (uint32_t)kd + (uint32_t)piece(R)) * 2u : GRP_OOB;
         }
     };
     auto issue = [&](int slot) {
@@ -340,7 +342,7 @@ __device__ __forceinline__ void grp_run(const mm_bf16_mm_args &a) {
         const int k0 = ic * KB;
 #pragma unroll
         for (int u = 0; u < sp::W_LPW; u++)
-            lds_dma16_buf_nt(wo[u] != OOB && k0 + piece(wload_row(u)) < kd ? wo[u] + (uint32_t)(2 * k0) : OOB,
+            lds_dma16_buf_nt(wo[u] != GRP_OOB && k0 + piece(wload_row(u)) < kd ? wo[u] + (uint32_t)(2 * k0) : GRP_OOB,
                              wup(u) ? wr[GU ? 1 : 0] : wr[0], sb + (uint32_t)(u * 1024));
         if (advance()) set_issue(tile_at(it));
     };
@@ -473,7 +475,7 @@ __device__ __forceinline__ void grp_run(const mm_bf16_mm_args &a) {
             nch = (a.seg[cur.si].Kd + KB - 1) / KB;
             cc = 0;
             zero();
-        } else if (cc % (FLUSH / KB) == 0) {
+        } else if (cc % (GRP_FLUSH / KB) == 0) {
             flush();
         }
     }
@@ -481,7 +483,7 @@ __device__ __forceinline__ void grp_run(const mm_bf16_mm_args &a) {
 }
 
 #define GRP_KERNEL(name, BM, GU)                                                            \
-    extern "C" __global__ __launch_bounds__((MMW + 1) * MM_WAVE, 1) void name(mm_bf16_mm_args a) { grp_run<BM, GU>(a); }
+    extern "C" __global__ __launch_bounds__((GRP_MMW + 1) * MM_WAVE, 1) void name(mm_bf16_mm_args a) { grp_run<BM, GU>(a); }
 GRP_KERNEL(mm_bf16_gu_16, 16, true)
 GRP_KERNEL(mm_bf16_gu_32, 32, true)
 GRP_KERNEL(mm_bf16_gu_64, 64, true)
