@@ -68,6 +68,8 @@ static const struct {
     [K_MLA_ROPE_QPREP] = {"mm_mla_rope_qprep", MOD_MLA},
     [K_MLA_ATTN] = {"mm_mla_attn", MOD_MLA},
     [K_MLA_ATTN_ROWS] = {"mm_mla_attn_rows", MOD_MLA},
+    [K_MLA_EXPAND] = {"mm_mla_expand", MOD_MLA},
+    [K_MLA_ATTN_X] = {"mm_mla_attn_expanded", MOD_MLA},
     [K_MLA_COMBINE] = {"mm_mla_combine", MOD_MLA},
     [K_MLA_UV] = {"mm_mla_uv", MOD_MLA},
     [K_MLA_QPREP_W] = {"mm_mla_qprep_w", MOD_MLA},
@@ -185,6 +187,11 @@ int mm_ctx_create(int device, mm_ctx **out) {
         const char *r4 = getenv("MLAMOE_MLA_ROWS4");
         c->mla_rows4 = !(r4 && r4[0] == '0');
     }
+    /* MLAMOE_MLA_EXPAND_MIN overrides the rows of one sequence from which an
+     * engine step's attention is expanded (0: never) */
+    c->mla_expand_min = MM_MLA_EXPAND_MIN;
+    ev = getenv("MLAMOE_MLA_EXPAND_MIN");
+    if (ev && *ev) c->mla_expand_min = atoi(ev);
     ev = getenv("MLAMOE_MLA_PART_MAX");
     if (ev && *ev && atoll(ev) > 0) c->mla_part_max = (size_t)atoll(ev);
     /* MLAMOE_MOE_T_CHUNK lowers the rows of one MoE forward pass (longer

@@ -39,8 +39,15 @@ struct mm_engine {
                                   planes [2, rows, n]: the projections' operands */
     int32_t *d_io;             /* device [IO_ARRAYS][max_rows]: see IO_* */
     int32_t *h_io;             /* pinned host, same layout */
+    int32_t *xt_h, *xt_d;      /* tile tables of a step's expanded attention (pinned host,
+                                  device): XT_MAX key tiles, then as many row tiles */
     int32_t *last_pos;         /* [max_batch] host: a step's check of its rows' positions */
 };
+
+/* Tiles of either kind a step's expanded attention may have (its sequences
+ * past that take the absorbed form): 131,072 keys. */
+#define XT_MAX 1024
+#define XT_BYTES (XT_MAX * (4 + 5) * sizeof(int32_t))
 
 /* the per-row arrays of a step, device and pinned host */
 enum { IO_TOK, IO_POS, IO_LEN, IO_SLOT, IO_WANT, IO_NEXT, IO_ARRAYS };
@@ -56,6 +63,8 @@ void mm_engine_destroy(mm_engine *e) {
     void *dev[] = {e->x, e->xn, e->q, e->ctxo, e->g, e->u, e->d_io, e->fcomp, e->xn_hl, e->ctx_hl};
     for (size_t i = 0; i < sizeof(dev) / sizeof(dev[0]); i++)
         if (dev[i]) hipFree(dev[i]);
+    if (e->xt_d) hipFree(e->xt_d);
+    if (e->xt_h) hipHostFree(e->xt_h);
     if (e->h_io) hipHostFree(e->h_io);
     free(e->last_pos);
     free(e->lcap);
@@ -166,6 +175,7 @@ int mm_engine_create(mm_ctx *c, const mm_engine_config *cfg, mm_engine **out) {
         {(void **)&e->ctxo, MR * (size_t)g->n_heads * g->v_head_dim * 4},
         {(void **)&e->g, MR * DI * 4}, {(void **)&e->u, MR * DI * 4},
         {(void **)&e->d_io, IO_ARRAYS * MR * 4},
+        {(void **)&e->xt_d, XT_BYTES},
         {(void **)&e->fcomp, (size_t)MM_SKINNY_T * KVD * 4},
         {(void **)&e->xn_hl, (size_t)MM_SKINNY_T * H * 4},
         {(void **)&e->ctx_hl, (size_t)MM_SKINNY_T * g->n_heads * g->v_head_dim * 4}};
@@ -174,7 +184,8 @@ int mm_engine_create(mm_ctx *c, const mm_engine_config *cfg, mm_engine **out) {
             mm_engine_destroy(e);
             return mm_fail(MM_ERR_NOMEM, "mm_engine_create: step buffers for %zu rows", MR);
         }
-    if (hipHostMalloc((void **)&e->h_io, IO_ARRAYS * MR * 4, 0) != hipSuccess) {
+    if (hipHostMalloc((void **)&e->h_io, IO_ARRAYS * MR * 4, 0) != hipSuccess ||
+        hipHostMalloc((void **)&e->xt_h, XT_BYTES, 0) != hipSuccess) {
         mm_engine_destroy(e);
         return mm_fail(MM_ERR_NOMEM, "mm_engine_create: pinned host buffer");
     }
@@ -287,8 +298,89 @@ static int dense_ffn(mm_engine *e, const mm_engine_layer *L, int B) {
     return mm_matmul_bf16_dev(c, e->x, e->g, L->dense_down, H, DI, B, MM_MATMUL_ACCUMULATE);
 }
 
+/* The rows of a step whose attention is expanded: runs of at least
+ * mla_expand_min rows of one slot at consecutive positions, and one per
+ * MM_MLA_EXPAND_KEYS keys, as long as their expanded keys fit the cap on a
+ * launch's attention scratch. */
+typedef struct {
+    int nkt, nqt, nblk;        /* tiles in xt_h, expanded 32-key blocks */
+    int n_abs, *abs;           /* the other rows: [first, end) pairs */
+} step_plan;
+
+static int by_len_desc(const void *a, const void *b) {
+    const int32_t *x = a, *y = b;
+    return (y[2] + y[1]) - (x[2] + x[1]);
+}
+
+static int plan_step(mm_engine *e, int R, step_plan *p) {
+    const mm_ctx *c = e->c;
+    const int MR = e->max_rows;
+    const int32_t *slot = e->h_io + IO_SLOT * MR, *pos = e->h_io + IO_POS * MR;
+    /* (up to MM_SKINNY_T rows the cache append waits for the absorbed queries'
+     * launch, and o_proj reads the pairs that the absorbed form writes) */
+    const int on = c->mla_expand_min > 0 && mm_mla_can_expand(c) && R > MM_SKINNY_T;
+    int32_t *kt = e->xt_h, *qt = e->xt_h + 4 * XT_MAX;
+    memset(p, 0, sizeof(*p));
+    if (!(p->abs = malloc((size_t)R * 2 * sizeof(int)))) return mm_fail(MM_ERR_NOMEM, "mm_engine_step: malloc");
+    for (int r = 0, n; r < R; r += n) {
+        n = 1;
+        while (r + n < R && slot[r + n] == slot[r] && pos[r + n] == pos[r] + n) n++;
+        const int len = pos[r] + n, nb = (len + 31) / 32;
+        const int k = (len + MM_MLA_XKEYS - 1) / MM_MLA_XKEYS, q = (n + MM_MLA_XROWS - 1) / MM_MLA_XROWS;
+        if (!on || n < c->mla_expand_min || len > MM_MLA_EXPAND_KEYS * n || p->nkt + k > XT_MAX || p->nqt + q > XT_MAX ||
+            (size_t)(p->nblk + nb) * c->mla.n_heads * MM_MLA_XBLK > c->mla_part_max) {
+            if (p->n_abs && p->abs[2 * p->n_abs - 1] == r) {
+                p->abs[2 * p->n_abs - 1] = r + n;
+            } else {
+                p->abs[2 * p->n_abs] = r;
+                p->abs[2 * p->n_abs++ + 1] = r + n;
+            }
+            continue;
+        }
+        for (int i = 0; i < k; i++) {
+            int32_t *t = kt + 4 * p->nkt++;
+            t[0] = slot[r];
+            t[1] = MM_MLA_XKEYS * i;
+            t[2] = len;
+            t[3] = p->nblk;
+        }
+        for (int i = 0; i < q; i++) {
+            int32_t *t = qt + 5 * p->nqt++;
+            t[0] = r + MM_MLA_XROWS * i;
+            t[1] = n - MM_MLA_XROWS * i < MM_MLA_XROWS ? n - MM_MLA_XROWS * i : MM_MLA_XROWS;
+            t[2] = pos[r] + MM_MLA_XROWS * i;
+            t[3] = slot[r];
+            t[4] = p->nblk;
+        }
+        p->nblk += nb;
+    }
+    /* Longest rows first, so that the last blocks to start are the shortest --
+     * but the second tile of each CU (two blocks share one, and 256 / n_heads
+     * tiles give every CU its first) shortest first: beside the longest. */
+    qsort(qt, (size_t)p->nqt, 5 * sizeof(int32_t), by_len_desc);
+    const int s = 256 / c->mla.n_heads;
+    for (int i = s, j = (p->nqt < 2 * s ? p->nqt : 2 * s) - 1; i < j; i++, j--) {
+        int32_t t[5];
+        memcpy(t, qt + 5 * i, sizeof(t));
+        memcpy(qt + 5 * i, qt + 5 * j, sizeof(t));
+        memcpy(qt + 5 * j, t, sizeof(t));
+    }
+    return MM_OK;
+}
+
+/* Every group of 4 of the rows [r0, r1) in one slot (a prompt's positions):
+ * the absorbed attention reads each group's keys once. */
+static int rows_by_4(const int32_t *slot, int r0, int r1) {
+    if (r1 - r0 < 2) return 0;
+    for (int r = r0; r < r1; r++)
+        if (slot[r] != slot[r0 + ((r - r0) & ~3)]) return 0;
+    return 1;
+}
+
 /* One step over R rows (h_io filled: tokens, positions, slots; want rows):
  * embedding, every layer over all rows, the LM head over the wanted rows. */
+static int run_planned(mm_engine *e, int R, int n_want, int32_t *next, float *logits, const step_plan *p);
+
 static int engine_run(mm_engine *e, int R, int n_want, int32_t *next, float *logits) {
     mm_ctx *c = e->c;
     const mm_engine_config *f = &e->cfg;
@@ -317,13 +409,24 @@ static int engine_run(mm_engine *e, int R, int n_want, int32_t *next, float *log
         if (w < 0 || w >= R || (j > 0 && w <= hio[IO_WANT * MR + j - 1]))
             return mm_fail(MM_ERR_INVALID, "mm_engine_step: want_rows must ascend within [0, %d)", R);
     }
-    /* every group of 4 rows in one slot (a prefill's positions): the
-     * attention reads each group's keys once */
-    int rows4 = R > 1;
-    for (int r = 0; r < R && rows4; r++) rows4 = hio[IO_SLOT * MR + r] == hio[IO_SLOT * MR + (r & ~3)];
     int st = mm_engine_reserve(e, kvmax);
     if (st) return st;
     if ((st = mm_set_device(c))) return st;
+    step_plan p;
+    if (!(st = plan_step(e, R, &p))) st = run_planned(e, R, n_want, next, logits, &p);
+    free(p.abs);
+    return st;
+}
+
+static int run_planned(mm_engine *e, int R, int n_want, int32_t *next, float *logits, const step_plan *p) {
+    mm_ctx *c = e->c;
+    const mm_engine_config *f = &e->cfg;
+    const int MR = e->max_rows;
+    int32_t *hio = e->h_io;
+    int st;
+    const int NH = c->mla.n_heads, QD = NH * (c->mla.qk_nope_head_dim + c->mla.qk_rope_head_dim);
+    if (p->nqt)
+        MM_HIP(hipMemcpyAsync(e->xt_d, e->xt_h, XT_BYTES, hipMemcpyHostToDevice, c->stream));
     int32_t *d_tok = e->d_io + IO_TOK * MR, *d_pos = e->d_io + IO_POS * MR;
     int32_t *d_len = e->d_io + IO_LEN * MR, *d_slot = e->d_io + IO_SLOT * MR;
     int32_t *d_want = e->d_io + IO_WANT * MR, *d_next = e->d_io + IO_NEXT * MR;
@@ -345,10 +448,20 @@ static int engine_run(mm_engine *e, int R, int n_want, int32_t *next, float *log
                                     fuse ? e->fcomp : NULL,
                                     fuse ? &ra : NULL)))
             return st;
-        if ((st = mm_mla_decode_rows(c, l, R, e->q, e->cache[l], e->lcap[l], d_slot, d_len, kvmax,
-                                     e->ctxo, NULL, NULL, NULL, fuse ? &ra : NULL,
-                                     hl_rows(e, R) ? e->ctx_hl : NULL, rows4)))
+        if (p->nqt && (st = mm_mla_expanded_rows(c, l, e->q, e->cache[l], e->lcap[l], e->xt_d, p->nkt,
+                                                 e->xt_d + 4 * XT_MAX, p->nqt, p->nblk, e->ctxo)))
             return st;
+        for (int i = 0; i < p->n_abs; i++) {
+            const int r0 = p->abs[2 * i], n = p->abs[2 * i + 1] - r0;
+            int kvlen = 1;     /* the range's longest context */
+            for (int r = r0; r < r0 + n; r++)
+                if (hio[IO_LEN * MR + r] > kvlen) kvlen = hio[IO_LEN * MR + r];
+            if ((st = mm_mla_decode_rows(c, l, n, e->q + (size_t)r0 * QD, e->cache[l], e->lcap[l], d_slot + r0,
+                                         d_len + r0, kvlen, e->ctxo + (size_t)r0 * NH * c->mla.v_head_dim, NULL,
+                                         NULL, NULL, fuse ? &ra : NULL, hl_rows(e, R) ? e->ctx_hl : NULL,
+                                         rows_by_4(hio + IO_SLOT * MR, r0, r0 + n))))
+                return st;
+        }
         const int dense = l < f->first_k_dense;
         if ((st = oproj_post_norm(e, L, R, dense))) return st;
         if (dense) {

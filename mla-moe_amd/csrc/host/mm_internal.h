@@ -45,6 +45,8 @@ typedef enum {
     K_MLA_ROPE_QPREP,
     K_MLA_ATTN,
     K_MLA_ATTN_ROWS,
+    K_MLA_EXPAND,
+    K_MLA_ATTN_X,
     K_MLA_COMBINE,
     K_MLA_UV,
     K_MLA_QPREP_W,
@@ -141,6 +143,8 @@ struct mm_ctx {
 
     int i8_tiled_min_t;         /* token count from which the tiled int8 GEMM is used */
     size_t mla_part_max;        /* attention chunk partials per launch (bytes) */
+    int mla_expand_min;         /* rows of one sequence from which a step's attention is
+                                   expanded (MLAMOE_MLA_EXPAND_MIN overrides) */
     int mla_rows4;              /* row groups sharing a sequence read its keys once
                                    (MLAMOE_MLA_ROWS4=0: per row, for comparisons) */
     int moe_t_chunk;            /* cap on the rows of one MoE forward pass (0: MM_MOE_T_CHUNK) */
@@ -265,6 +269,16 @@ int mm_mla_decode_rows(mm_ctx *ctx, int layer, int B, const float *q, const uint
                        int seq_stride, const int32_t *slots, const int32_t *kv_lens, int kv_len,
                        float *ctx_out, float *qabs, float *probs, float *clat,
                        const mm_mla_rope_args *rope, uint16_t *ctx_hl, int rows4);
+
+/* Attention of prompt rows in the expanded form (csrc/kernels/mla_expand.h):
+ * nkt 128-key tiles (slot, first key, length, first block each) expanded into
+ * nblk blocks, then nqt MM_MLA_XROWS-row tiles (first row, rows, first position, slot,
+ * first block each); both tables on the device.  mm_mla_can_expand: whether
+ * the configured head dimensions are served. */
+int mm_mla_can_expand(const mm_ctx *ctx);
+int mm_mla_expanded_rows(mm_ctx *ctx, int layer, const float *q, const uint16_t *cache, int seq_stride,
+                         const int32_t *ktiles, int nkt, const int32_t *qtiles, int nqt, int nblk,
+                         float *ctx_out);
 
 void mm_moe_release(mm_ctx *ctx);
 void mm_mla_release(mm_ctx *ctx);

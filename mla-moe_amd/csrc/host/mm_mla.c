@@ -228,6 +228,25 @@ static int decode_rows(mm_ctx *c, int layer, int B, const float *q, const uint16
                      (unsigned)((B + 31) / 32), 256, 0, &ca);
 }
 
+/* ---- expanded attention of prompt rows ------------------------------------------ */
+
+int mm_mla_can_expand(const mm_ctx *c) {
+    return c->mla.qk_nope_head_dim == MM_MLA_XD && c->mla.v_head_dim == MM_MLA_XD;
+}
+
+int mm_mla_expanded_rows(mm_ctx *c, int layer, const float *q, const uint16_t *cache, int seq_stride,
+                         const int32_t *ktiles, int nkt, const int32_t *qtiles, int nqt, int nblk,
+                         float *ctx_out) {
+    const int NH = c->mla.n_heads;
+    uint8_t *kv;
+    int st = mm_workspace(c, (size_t)nblk * NH * MM_MLA_XBLK, (void **)&kv);
+    if (st) return st;
+    mm_mla_expand_args ea = {cache, c->mla_kvb[layer], kv, ktiles, seq_stride, NH};
+    if ((st = mm_launch(c, K_MLA_EXPAND, (unsigned)NH, 2, (unsigned)nkt, 512, MM_MLA_XEXP_LDS, &ea))) return st;
+    mm_mla_xattn_args xa = {q, cache, kv, qtiles, ctx_out, seq_stride, NH, c->mla.softmax_scale};
+    return mm_launch(c, K_MLA_ATTN_X, (unsigned)nqt * (unsigned)NH, 1, 1, 256, MM_MLA_XATTN_LDS, &xa);
+}
+
 /* ---- decode front ---------------------------------------------------------- */
 
 /* build_rope_inv_freq (src/model_load.c:299-325), step for step in fp32. */

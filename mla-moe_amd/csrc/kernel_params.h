@@ -437,6 +437,39 @@ typedef struct {
     uint16_t *ctx_hl;         /* or 0: ctx also as bf16 hi/lo planes [2, B, NH * VHD] */
 } mm_mla_combine_args;
 
+/* ---- MLA attention of a prompt's rows, expanded (mla_expand.h) --------------- */
+#define MM_MLA_XD 128             /* qk_nope and v head dims served */
+#define MM_MLA_XBLK 32768         /* bytes of 32 keys' K and V pairs of one head */
+#define MM_MLA_XROWS 64           /* rows per attention block */
+#define MM_MLA_XKEYS 128          /* keys per expanding block */
+/* A step's rows of one sequence are attended in the expanded form from
+ * MM_MLA_EXPAND_MIN rows on, and from one row per MM_MLA_EXPAND_KEYS keys:
+ * fewer do not pay for expanding the keys, and are too few blocks for long
+ * chains (4-layer step, absorbed and expanded: 65 rows 1035 and 1005 us, after
+ * 1,000 positions 1150 and 1147, after 4,000 1316 and 1586; 192 rows after
+ * 4,000 1957 and 1990, 256 rows 2170 and 1898, 512 rows 2946 and 2122). */
+#define MM_MLA_EXPAND_MIN 65
+#define MM_MLA_EXPAND_KEYS 20
+#define MM_MLA_XNS 2              /* chunks of latent values in an expanding block's ring */
+#define MM_MLA_XEXP_LDS (MM_MLA_XNS * 32768)
+#define MM_MLA_XATTN_LDS (2 * (MM_MLA_XBLK + 32 * 128))
+typedef struct {
+    const uint16_t *cache;    /* [sequences, seq_stride, KVL + QKR] */
+    const uint16_t *kv_b;     /* [NH, W_UK 128 rows | W_UV 128 rows, KVL] */
+    uint8_t *kv;              /* [blocks][NH] blocks of MM_MLA_XBLK bytes */
+    const int32_t *tiles;     /* per 128 keys: slot, first key, sequence length, first block */
+    int seq_stride, NH;
+} mm_mla_expand_args;
+typedef struct {
+    const float *q;           /* [R, NH, 128 + QKR] */
+    const uint16_t *cache;
+    const uint8_t *kv;
+    const int32_t *tiles;     /* per 64 rows: first row, rows, first position, slot, first block */
+    float *ctx;               /* [R, NH * 128] */
+    int seq_stride, NH;
+    float scale;
+} mm_mla_xattn_args;
+
 /* ---- dense bf16 matmul --------------------------------------------------------- */
 /* y[t, d] (=|+=) sum_i x[t, i] * W[d, i]; W bf16 row-major [d_out, n_in].  x
  * is first converted to bf16 rows of a padded stride kp (a multiple of 64,

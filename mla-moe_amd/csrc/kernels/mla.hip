@@ -863,6 +863,8 @@ extern "C" __global__ __launch_bounds__(AW * MM_WAVE) void mm_mla_attn_rows(mm_m
     }
 }
 
+#include "mla_expand.h"
+
 /* Merge the chunk partials of (head h, sequence b): clat = sum_c w_c O_c / l
  * with w_c = e^(m_c - m); also turns the debug scores into probabilities.
  * grid (NH, B, Z) with Z = 1 or KVL / 128, 256 threads: block z owns the

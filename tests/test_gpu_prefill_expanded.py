@@ -1,0 +1,84 @@
+"""Prefill attention in the expanded form (keys and values per head, the rows
+of a prompt in 128-row tiles): prompts at the edges of its tiles, several
+prompts of unequal length in one step, a chunk after earlier positions, and
+decode rows beside them, against the absorbed form of the same engine.
+
+Both forms carry fp32 operands as bf16 pairs (relative error below 2^-17 per
+operand, random) and read the same bf16 latent cache; one layer's appended
+row may then round differently in the next layer's cache (2^-9 of an
+element, rarely).  Logits agree to 2e-4 of their norm (measured 3e-5)."""
+import numpy as np
+import pytest
+
+import mlamoe
+from mlamoe import synth
+from mlamoe.engine import Engine
+
+pytestmark = pytest.mark.gpu
+
+CFG = dict(n_layers=2, first_dense=2, H=256, NH=4, QKN=128, QKR=64, KVL=512, VHD=128, dense_inter=128, E=4,
+           n_shared=1, K=2, I=64, vocab=300, router_sigmoid=0, norm_topk=0, routed_scaling=1.0, rms_eps=1e-6)
+
+
+@pytest.fixture(scope="module")
+def model():
+    c = CFG
+    return synth.model(4321, c["n_layers"], c["first_dense"], c["H"], c["NH"], c["QKN"], c["QKR"], c["KVL"], c["VHD"],
+                       c["dense_inter"], c["E"], c["I"], c["n_shared"], c["vocab"])
+
+
+def logits(model, steps, monkeypatch, expand_min):
+    """Each step: a list of (slot, first position, rows).  All rows' logits."""
+    monkeypatch.setenv("MLAMOE_MLA_EXPAND_MIN", str(expand_min))
+    rng = np.random.default_rng(5)
+    toks = rng.integers(0, CFG["vocab"], (8, 2048)).astype(np.int32)
+    out = []
+    with mlamoe.Context(0) as ctx:
+        eng = Engine.from_host(ctx, CFG, model, mlamoe.rope_inv_freq(64, 10000.0), max_batch=8, max_seq=1200,
+                               max_rows=2048)
+        try:
+            for st in steps:
+                rows = [(s, p0 + i) for s, p0, n in st for i in range(n)]
+                sl, ps = (np.array(a, np.int32) for a in zip(*rows))
+                _, lg = eng.step_rows(sl, toks[sl, ps], ps, np.arange(len(rows)), want_logits=True)
+                out.append(lg)
+        finally:
+            eng.close()
+    return np.concatenate(out).astype(np.float64)
+
+
+@pytest.mark.parametrize("steps", [
+    [[(0, 0, 128)]], [[(0, 0, 129)]], [[(3, 0, 161)]], [[(0, 0, 65)]], [[(1, 0, 1023)]],
+    [[(0, 0, 300), (1, 0, 50), (2, 0, 128), (5, 0, 255)]],                  # unequal prompts (50: absorbed)
+    [[(0, 0, 37)], [(0, 37, 200), (1, 0, 130)], [(0, 237, 1), (1, 130, 1), (2, 0, 140)]],   # chunks, decode rows
+    [[(0, 0, 31)], [(0, 31, 66)], [(0, 97, 513)]],
+    [[(0, 0, 1000), (1, 0, 1000)], [(0, 1000, 100), (1, 1000, 150)]],
+], ids=lambda s: "-".join("+".join(str(n) for _, _, n in st) for st in s))
+def test_expanded_agrees_with_absorbed(model, monkeypatch, steps):
+    a = logits(model, steps, monkeypatch, 65)
+    b = logits(model, steps, monkeypatch, 0)
+    err = np.linalg.norm(a - b) / np.linalg.norm(b)
+    worst = np.max(np.linalg.norm(a - b, axis=1) / np.linalg.norm(b, axis=1))
+    print(f"{steps}: {err:.2e}, worst row {worst:.2e}", flush=True)
+    assert err < 2e-4 and worst < 2e-3
+    assert err > 0                       # another form did run
+
+
+def test_expanded_against_oracle(model, monkeypatch, oracle):
+    """Every position of a 150-token prompt against the reference's forward."""
+    got = logits(model, [[(0, 0, 150)]], monkeypatch, 128)
+    toks = np.random.default_rng(5).integers(0, CFG["vocab"], (8, 2048)).astype(np.int32)[0, :150]
+    ref = oracle.model_logits(CFG, model, toks, mlamoe.rope_inv_freq(64, 10000.0))
+    err = np.max(np.abs(got - ref), axis=1) / np.max(np.abs(ref), axis=1)
+    print(f"worst normwise logits error {err.max():.2e}", flush=True)
+    assert err.max() < 2e-3              # the bar of the other prefill tests (bf16 cache, fp32 in the reference)
+
+
+def test_scratch_cap_falls_back(model, monkeypatch):
+    """Prompts whose expanded keys do not fit the attention scratch cap take
+    the absorbed form: here the second of two."""
+    monkeypatch.setenv("MLAMOE_MLA_PART_MAX", str(40 * 4 * 32768))     # 40 blocks of 4 heads
+    steps = [[(0, 0, 1000), (1, 0, 600)]]
+    a = logits(model, steps, monkeypatch, 128)
+    b = logits(model, steps, monkeypatch, 0)
+    assert np.linalg.norm(a - b) < 2e-4 * np.linalg.norm(b)
