@@ -55,39 +55,42 @@ int mm_lm_head_dev(mm_ctx *c, int B, const float *x, const uint16_t *norm, float
     /* workspace: xb [B, hidden] (GEMM path), logits [B, vocab] when not
      * returned, GEMM staging, argmax partials */
     const size_t rpb = 4 * MM_GEMV_RPW;           /* GEMV rows per block per turn */
-    const size_t nb = gemv ? (((size_t)vocab + rpb - 1) / rpb < MM_LM_GEMV_BLOCKS
-                                  ? ((size_t)vocab + rpb - 1) / rpb : MM_LM_GEMV_BLOCKS)
-                           : 0;
+    const int mfma = !gemv && B <= 64 && hidden % 64 == 0 && hidden <= MM_LMG_KMAX &&
+                     (uintptr_t)x % 16 == 0 && (uintptr_t)norm % 16 == 0;
+    /* blocks that write argmax partials themselves */
+    const size_t units = gemv ? ((size_t)vocab + rpb - 1) / rpb : ((size_t)vocab + 15) / 16;
+    const size_t nbmax = gemv ? MM_LM_GEMV_BLOCKS : MM_LMG_BLOCKS;
+    const size_t nb = units < nbmax ? units : nbmax;
     const size_t o_xb = 0, n_xb = gemv ? 0 : al256((size_t)B * hidden * 4);
     const size_t o_lg = o_xb + n_xb, n_lg = logits ? 0 : al256((size_t)B * vocab * 4);
     const size_t o_gm = o_lg + n_lg, n_gm = gemv ? 0 : al256(mm_gemm_bf16_ws_bytes(B, hidden, vocab, 0));
     const size_t o_am = o_gm + n_gm;
-    const size_t n_am = gemv ? 2 * al256((size_t)B * nb * 4) : argmax_ws(B, vocab);
+    const size_t n_am = gemv || mfma ? 2 * al256((size_t)B * nb * 4) : argmax_ws(B, vocab);
     char *ws;
     if ((st = mm_workspace(c, o_am + n_am, (void **)&ws))) return st;
     float *lg = logits ? logits : (float *)(ws + o_lg);
-    if (gemv) {
-        /* one pass: norm, logits, per-block argmax partials; then the final
-         * reduction over the nb partials of each token */
+    if (gemv || mfma) {
+        /* the logits kernel leaves its blocks' argmax partials: then only the
+         * final reduction over the nb partials of each token */
         float *pv = (float *)(ws + o_am);
         int32_t *pi = (int32_t *)(ws + o_am + al256((size_t)B * nb * 4));
-        mm_lm_gemv_args ga = {x, norm, eps, lm_head, lg, pv, pi, B, vocab, hidden};
-        const mm_kernel_id id = B <= 1 ? K_LM_GEMV1 : B <= 2 ? K_LM_GEMV2 : K_LM_GEMV4;
-        if ((st = mm_launch(c, id, (unsigned)nb, 1, 1, 256, 0, &ga))) return st;
+        if (gemv) {   /* the norm too */
+            mm_lm_gemv_args ga = {x, norm, eps, lm_head, lg, pv, pi, B, vocab, hidden};
+            const mm_kernel_id id = B <= 1 ? K_LM_GEMV1 : B <= 2 ? K_LM_GEMV2 : K_LM_GEMV4;
+            if ((st = mm_launch(c, id, (unsigned)nb, 1, 1, 256, 0, &ga))) return st;
+        } else {
+            /* the norm writes bf16 hi/lo planes (the same bytes as xb's fp32)
+             * for the logits GEMM's direct-to-LDS ring */
+            uint16_t *xhl = (uint16_t *)(ws + o_xb);
+            mm_rmsnorm_hl_args rh = {x, norm, xhl, hidden, eps};
+            if ((st = mm_launch(c, K_RMSNORM_HL, (unsigned)B, 1, 1, 256, 0, &rh))) return st;
+            mm_lm_gemm_args ga = {xhl, lm_head, lg, pv, pi, B, vocab, hidden};
+            if ((st = mm_launch(c, K_LM_GEMM, (unsigned)nb, 1, 1, MM_LMG_THREADS,
+                                (size_t)MM_LMG_NSW * MM_LMG_WB + (size_t)MM_LMG_NSX * MM_LMG_XB, &ga)))
+                return st;
+        }
         mm_argmax_args fa = {lg, tokens, pv, pi, vocab, B, (int)nb};
         return mm_launch(c, K_ARGMAX_FINAL, (unsigned)B, 1, 1, 256, 0, &fa);
-    }
-    if (B <= 64 && hidden % 64 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)norm % 16 == 0) {
-        /* the norm writes bf16 hi/lo planes (the same bytes as xb's fp32)
-         * for the logits GEMM's direct-to-LDS ring */
-        uint16_t *xhl = (uint16_t *)(ws + o_xb);
-        mm_rmsnorm_hl_args rh = {x, norm, xhl, hidden, eps};
-        if ((st = mm_launch(c, K_RMSNORM_HL, (unsigned)B, 1, 1, 256, 0, &rh))) return st;
-        mm_lm_gemm_args lg_a = {xhl, lm_head, lg, B, vocab, hidden};
-        if ((st = mm_launch(c, K_LM_GEMM, (unsigned)((vocab + MM_LMG_BN - 1) / MM_LMG_BN), 1, 1, 256,
-                            (size_t)MM_LMG_NS * MM_LMG_STAGE, &lg_a)))
-            return st;
-        return argmax_launch(c, B, lg, vocab, tokens, ws + o_am);
     }
     float *xb = (float *)(ws + o_xb);
     mm_rmsnorm_args ra = {x, norm, xb, hidden, eps};

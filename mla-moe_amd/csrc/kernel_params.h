@@ -603,15 +603,24 @@ typedef struct {
 } mm_rmsnorm_hl_args;
 
 /* Logits GEMM for MM_LM_NB < T <= 64 rows: y[T, N] = x . W^T with x given
- * as bf16 hi/lo planes; MM_LMG_BN columns per block. */
-#define MM_LMG_BN 256
-#define MM_LMG_NS 3                                  /* ring stages (two chunks ahead) */
-#define MM_LMG_STAGE (MM_LMG_BN * 128 + 2 * 64 * 128) /* LDS bytes per stage: W, x hi, x lo */
+ * as bf16 hi/lo planes, and the best logit of each block's columns.  At most
+ * MM_LMG_BLOCKS blocks, none without a 16-column unit. */
+#define MM_LMG_BLOCKS 256                            /* one per CU */
+#define MM_LMG_THREADS 704                           /* 8 multiplying, 3 loading waves */
+#define MM_LMG_MU 7                                  /* 16-column units per pass */
+#define MM_LMG_WC 4                                  /* 64-wide K chunks per W ring stage */
+#define MM_LMG_NSW 2                                 /* W ring stages */
+#define MM_LMG_NSX 3                                 /* x ring stages, one chunk each */
+#define MM_LMG_WB (MM_LMG_MU * 16 * 128 * MM_LMG_WC) /* LDS bytes per stage: W */
+#define MM_LMG_XB (2 * 64 * 128)                     /* x hi, x lo */
+#define MM_LMG_KMAX (1 << 22)                        /* byte offsets in 32 bits */
 typedef struct {
     const uint16_t *xhl;     /* [2, T, K] */
     const uint16_t *w;       /* [N, K] bf16 */
-    float *y;                /* [T, N] */
-    int T, N, K;             /* K a multiple of 64 */
+    float *y;                /* [T, N], 16-byte aligned */
+    float *part_v;           /* [T, blocks] each block's best logit */
+    int32_t *part_i;         /* [T, blocks] its column */
+    int T, N, K;             /* K a multiple of 64, at most MM_LMG_KMAX */
 } mm_lm_gemm_args;
 
 #define MM_ARGMAX_SEG 1024       /* row elements per argmax segment (block) */

@@ -105,6 +105,10 @@ __device__ __forceinline__ rsrc_t raw_rsrc(const void *base, uint32_t num_record
     r.y = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) & 0xffffu;
     r.z = num_records;
     r.w = 0x00020000u;
+    /* 5 wait states between a vector instruction that writes a scalar
+     * register (readfirstlane) and a buffer access that reads it: the
+     * compiler does not see the accesses written as inline assembly */
+    asm("s_nop 4" : "+s"(r));
     return r;
 }
 

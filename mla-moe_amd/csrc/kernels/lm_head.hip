@@ -15,10 +15,12 @@
  *   mm_lm_gemv   for up to MM_LM_NB tokens: rmsnorm, logits (every weight
  *                row read once: HBM-bound, 2 bytes per weight) and per-wave
  *                argmax partials in one pass (the GEMV core of gemv.h)
+ *   mm_rmsnorm_hl + mm_lm_gemm  for up to 64 tokens: the same split, logits on
+ *                the matrix cores
  *   mm_rmsnorm   one block per token (the GEMM path for more tokens)
  *   mm_argmax_part / mm_argmax_final   segments of every row in parallel
- *                (the GEMV path writes its partials itself), then one block
- *                per row over the partials
+ *                (mm_lm_gemv and mm_lm_gemm write their partials themselves),
+ *                then one block per row over the partials
  */
 #include "gemv.h"
 
@@ -277,138 +279,255 @@ extern "C" __global__ __launch_bounds__(256) void mm_argmax_final(mm_argmax_args
 
 /* ---- logits GEMM for 5..64 rows ----------------------------------------------
  *
- * y[T, N] = x . W^T for the LM head's batch rows: MM_LMG_BN = 256 vocabulary
- * rows (output columns) per block, one block per CU (4 waves, wave w owns
- * columns 64 w .. + 63 for all 64 token rows: 4 x 4 tiles of
- * v_mfma_f32_16x16x32_bf16, x as the A operand and W as B, each fp32 x a
- * bf16 hi/lo pair as in mm_gemm_skinny, the same MFMA sequence per output:
- * per 32-wide K step the hi product, then the lo product).
+ * y[T, N] = x . W^T for the LM head's batch rows, and every block's best
+ * logit per token for the argmax.  Bound by the weight stream (2 N K bytes).
  *
- * Both operands go global -> LDS by direct loads into a ring of
- * MM_LMG_NS stages of one 64-wide K chunk (W: 256 rows x 128 B; x: the hi
- * and lo planes, 64 rows x 128 B each), two chunks ahead of their use.  The
- * skinny GEMM staged x through registers, so each wait for x -- an L2 hit
- * -- also waited for the weight loads issued before it (vector memory
- * counts complete in order) and the weight stream ran ~2 chunks deep:
- * 0.35 of HBM peak at the LM head.  Here every load in the loop belongs to
- * the ring, whose stages complete in the order they are consumed.
- * Measured against streaming W into registers four chunks deep with x alone
- * in the ring (one wave per SIMD): 114 against 161 us at 64 x 102400 x 2048.
+ * Persistent, one block per CU: the vocabulary's 16-column units are dealt out
+ * evenly in contiguous ranges (102400 columns: 25 units for each of 256
+ * blocks), and a block takes its range in equal passes of at most MM_LMG_MU
+ * units.  (One 256-column tile per block left 400 blocks on 256 CUs: the
+ * second turn filled 56% of them.)
  *
- * LDS rows are 128 B (8 pieces of 16 B); piece p of row r sits in slot
- * p ^ swz(r), so the 16 lanes of an MFMA operand read (16 consecutive rows,
- * one piece) hit 16 distinct 16-byte bank groups. */
-#define LMG_WB (MM_LMG_BN * 128)     /* W bytes per stage */
-#define LMG_LPW 12                   /* direct loads per wave per stage: 8 of W, 4 of x */
+ * Eight waves multiply, two load W, one loads x's bf16 hi/lo planes, into two
+ * LDS rings that run on across passes: W in stages of four 64-wide K chunks, x
+ * one chunk at a time.  A wave's vector memory operations complete in order,
+ * so a wave that loaded both operands could not wait for x (an L2 hit) without
+ * waiting for weights (HBM, wanted far ahead), and a multiplying wave that
+ * loaded any would wait behind its stores of y.  Loads of rows past the pass's
+ * columns or T are out of the buffer's range: no memory is read, zeros are
+ * staged.
+ *
+ * W streams faster in longer pieces of a row (loads alone, 64 x 102400 x 2048:
+ * 83 us in 128-byte pieces, 74 us in 512-byte pieces), which is why a pass is
+ * only 112 columns wide although x (512 KB) is then read from L2 four times
+ * per block: whole LM head 111.2 us, 112.5 us with two passes of 208 columns
+ * in 128-byte pieces, 147 us with a tile per block.
+ *
+ * Multiplying wave w owns units w % 4, w % 4 + 4, .. of the pass for 32 rows:
+ * v_mfma_f32_16x16x32_bf16 with W as the first operand, so that a lane holds 4
+ * consecutive columns of one row; per 32-wide K step every output takes its hi
+ * product, then its lo product (mm_gemm_skinny's sequence).  The operands of
+ * the next step are read during the current step's MFMAs.
+ *
+ * LDS rows are 16-byte pieces, piece p of row r in slot p ^ swz(r): the 16
+ * lanes of an operand read (16 consecutive rows, one piece) hit distinct
+ * 16-byte bank groups. */
+#define LMG_MMW 8                     /* multiplying waves: 4 over the units x 2 over the rows */
+#define LMG_WLD 2                     /* W-loading waves */
+#define LMG_PPR (8 * MM_LMG_WC)       /* 16-byte pieces per W row in LDS */
+#define LMG_RPL (MM_WAVE / LMG_PPR)   /* W rows per load */
+#define LMG_W_LPW (16 * MM_LMG_MU / LMG_RPL / LMG_WLD)   /* loads per W-loading wave per stage */
+#define LMG_X_LPW 16                  /* loads of the x-loading wave per chunk */
+#define LMG_UPW ((MM_LMG_MU + 3) / 4)   /* units per multiplying wave */
+#define LMG_GPW 2                     /* 16-row groups per multiplying wave */
+#define LMG_OOB 0xFFFFFFF0u           /* past every buffer range */
+static_assert(MM_LMG_THREADS == (LMG_MMW + LMG_WLD + 1) * MM_WAVE, "threads known to the host");
+static_assert(LMG_W_LPW * LMG_RPL * LMG_WLD == 16 * MM_LMG_MU && LMG_W_LPW * (MM_LMG_NSW - 1) < 64 && LMG_X_LPW * (MM_LMG_NSX - 1) < 64, "loads in flight: vmcnt");
 typedef __bf16 lmg_bf16x8 __attribute__((ext_vector_type(8)));
+typedef const __attribute__((address_space(3))) i32x4 *lmg_lds_cp;
 
-__device__ __forceinline__ int lmg_swz(int r) { return (r >> 1) & 7; }
+/* the slots' swizzle for rows of 16-byte pieces, 8 or more of them */
+__device__ __forceinline__ int lmg_swz(int r, int pieces) { return pieces == 8 ? (r >> 1) & 7 : r & 15; }
 
-extern "C" __global__ __launch_bounds__(256) void mm_lm_gemm(mm_lm_gemm_args a) {
-    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n0 = blockIdx.x * MM_LMG_BN;
-    const int K = a.K, T = a.T, N = a.N, nch = K / 64;
-    const int q = lane & 7;
-
-    /* direct loads of a chunk: W instruction 8 wave + u covers tile rows
-     * (columns) 8 (8 wave + u) .. + 7, x instruction 4 wave + u plane
-     * (4 wave + u) / 8, token rows 8 ((4 wave + u) % 8) .. + 7; lane l loads
-     * row + l / 8, slot q = l % 8, i.e. piece q ^ swz(row).  Rows past N or
-     * T load the last one (not stored). */
-    const uint16_t *wp[8], *xp[4];
+/* A loading wave: NI loads per stage, a stage being CPS 64-wide chunks of K;
+ * byte offsets vo[] within a buffer whose base moves one stage at a time, NS
+ * ring stages of `stage` bytes.  One barrier per chunk, as the multiplying
+ * waves have. */
+template <int NI, int NS, int CPS, bool NT, class F>
+__device__ __forceinline__ void lmg_load(int np, int nch, uint32_t lds0, uint32_t stage, F pass_of) {
+    const uint16_t *base;
+    uint32_t range, vo[NI];
+    const int nst = (nch + CPS - 1) / CPS, total = np * nst;
+    int ip = 0, is = 0, slot = 0;                  /* pass, stage and slot of the next issue */
+    auto issue = [&]() {
+        if (is == 0) pass_of(ip, base, range, vo);
+        const rsrc_t r = raw_rsrc(base + 64 * CPS * (size_t)is,
+                                  __builtin_amdgcn_readfirstlane(range - 128u * CPS * (uint32_t)is));
+        const uint32_t sb = lds0 + (uint32_t)slot * stage;
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
-        const int c = 8 * (8 * wave + u) + (lane >> 3);
-        wp[u] = a.w + (size_t)min(n0 + c, N - 1) * K + 8 * (q ^ lmg_swz(c));
-    }
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-        const int i = 4 * wave + u, r = 8 * (i & 7) + (lane >> 3);
-        xp[u] = a.xhl + (size_t)(i >> 3) * T * K + (size_t)min(r, T - 1) * K + 8 * (q ^ lmg_swz(r));
-    }
-    auto issue = [&](int c, int st) {
-        uint8_t *sb = lds + st * MM_LMG_STAGE;
-#pragma unroll
-        for (int u = 0; u < 8; u++) lds_dma16(wp[u] + 64 * c, sb + (8 * wave + u) * 1024);
-#pragma unroll
-        for (int u = 0; u < 4; u++) lds_dma16(xp[u] + 64 * c, sb + LMG_WB + (4 * wave + u) * 1024);
-    };
-
-    /* operand reads (bytes within a stage), K half s: A rows 16 g + l % 16,
-     * B rows (columns) 64 wave + 16 j + l % 16, piece 4 s + l / 16 */
-    uint32_t ao[2][4], bo[2][4];
-#pragma unroll
-    for (int s = 0; s < 2; s++) {
-        const int p = 4 * s + (lane >> 4);
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const int r = 16 * g + (lane & 15);
-            ao[s][g] = LMG_WB + r * 128 + 16 * (p ^ lmg_swz(r));
-            const int c = 64 * wave + 16 * g + (lane & 15);
-            bo[s][g] = c * 128 + 16 * (p ^ lmg_swz(c));
+        for (int u = 0; u < NI; u++) {
+            if (NT) lds_dma16_buf_nt(vo[u], r, sb + (uint32_t)u * 1024u);
+            else lds_dma16_buf(vo[u], r, sb + (uint32_t)u * 1024u);
         }
-    }
-    f32x4 acc[4][4];
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-#pragma unroll
-        for (int g = 0; g < 4; g++) acc[j][g] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-
-    const uint32_t l0 = lds_addr(lds);
-    issue(0, 0);
-    if (nch > 1) issue(1, 1);
-    for (int c = 0; c < nch; c++) {
-        /* chunk c landed: the loads of chunk c + 1 (issued after) may stay
-         * out; the barrier makes every wave's loads of chunk c visible and
-         * frees the stage of chunk c - 1 for chunk c + 2 */
-        if (c + 1 < nch) VMCNT_WAIT(LMG_LPW);
+        slot = slot + 1 == NS ? 0 : slot + 1;
+        if (++is == nst) {
+            is = 0;
+            ip++;
+        }
+    };
+#pragma unroll 1
+    for (int i = 0; i < NS - 1 && i < total; i++) issue();
+    int cs = 0;
+    for (int i = 0; i < total; i++) {
+        /* stage i landed: only the loads of the NS - 2 stages after it may be out */
+        if (i + NS - 2 < total) VMCNT_WAIT(NI * (NS - 2));
         else VMCNT_WAIT(0);
         __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-        if (c + 2 < nch) issue(c + 2, (c + 2) % MM_LMG_NS);
-        __builtin_amdgcn_sched_barrier(0);
-        const uint32_t sb = l0 + (uint32_t)((c % MM_LMG_NS) * MM_LMG_STAGE);
+        if (i + NS - 1 < total) issue();   /* into the slot of stage i - 1, read before the barrier */
+        for (int c = CPS * cs + 1; c < min(CPS * (cs + 1), nch); c++) __builtin_amdgcn_s_barrier();
+        cs = cs + 1 == nst ? 0 : cs + 1;
+    }
+}
+
+extern "C" __global__ __launch_bounds__(MM_LMG_THREADS, 1) void mm_lm_gemm(mm_lm_gemm_args a) {
+    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+    const int tid = threadIdx.x, lane = tid & (MM_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / MM_WAVE);
+    const int K = a.K, T = a.T, N = a.N, nch = K / 64;
+    const int nu = (N + 15) / 16;
+    /* (integer divisions run on the vector unit: back to scalars) */
+    const int ub = __builtin_amdgcn_readfirstlane((int)((int64_t)nu * blockIdx.x / gridDim.x));
+    const int un = __builtin_amdgcn_readfirstlane((int)((int64_t)nu * (blockIdx.x + 1) / gridDim.x)) - ub;
+    const int np = (un + MM_LMG_MU - 1) / MM_LMG_MU;
+    auto first = [&](int p) { return ub + __builtin_amdgcn_readfirstlane(un * p / np); };   /* first unit of pass p */
+    const uint32_t ldsw = lds_addr(lds), ldsx = ldsw + MM_LMG_NSW * MM_LMG_WB;
+
+    if (wave >= LMG_MMW + LMG_WLD) {   /* x: load i is plane i / 8, rows from 8 (i % 8) */
+        lmg_load<LMG_X_LPW, MM_LMG_NSX, 1, false>(
+            np, nch, ldsx, MM_LMG_XB, [&](int, const uint16_t *&base, uint32_t &range, uint32_t *vo) {
+                base = a.xhl;
+                range = 4u * (uint32_t)T * (uint32_t)K;
 #pragma unroll
-        for (int s = 0; s < 2; s++) {
-            i32x4 xa[4][2], wb[4];
+                for (int i = 0; i < LMG_X_LPW; i++) {
+                    const int r = 8 * (i & 7) + (lane >> 3);
+                    vo[i] = r < T ? 2u * (uint32_t)((i >> 3) * T + r) * (uint32_t)K + 16u * (uint32_t)((lane & 7) ^ lmg_swz(r, 8)) : LMG_OOB;
+                }
+            });
+    } else if (wave >= LMG_MMW) {
+        const int w0 = LMG_W_LPW * (wave - LMG_MMW);
+        lmg_load<LMG_W_LPW, MM_LMG_NSW, MM_LMG_WC, true>(
+            np, nch, ldsw + 1024u * (uint32_t)w0, MM_LMG_WB,
+            [&](int p, const uint16_t *&base, uint32_t &range, uint32_t *vo) {
+                const int n0 = 16 * first(p), cols = min(16 * first(p + 1), N) - n0;
+                base = a.w + (size_t)n0 * K;
+                range = 2u * (uint32_t)cols * (uint32_t)K;
 #pragma unroll
-            for (int g = 0; g < 4; g++) {
-                xa[g][0] = ds_read16(sb + ao[s][g]);
-                xa[g][1] = ds_read16(sb + ao[s][g] + 64 * 128);
-            }
+                for (int u = 0; u < LMG_W_LPW; u++) {
+                    const int r = LMG_RPL * (w0 + u) + lane / LMG_PPR;
+                    vo[u] = r < cols ? 2u * (uint32_t)r * (uint32_t)K + 16u * (uint32_t)(lane % LMG_PPR ^ lmg_swz(r, LMG_PPR)) : LMG_OOB;
+                }
+            });
+    }
+
+    const int l16 = lane & 15, g4 = lane >> 4;
+    const int wu = wave & 3, g0 = wave / 4 * LMG_GPW;   /* a multiplying wave's units (mod 4), 16-row groups */
+    float bv[LMG_GPW];
+    int bi[LMG_GPW];
 #pragma unroll
-            for (int j = 0; j < 4; j++) wb[j] = ds_read16(sb + bo[s][j]);
-            asm volatile("s_waitcnt lgkmcnt(0)"
-                         : "+v"(xa[0][0]), "+v"(xa[0][1]), "+v"(xa[1][0]), "+v"(xa[1][1]),
-                           "+v"(xa[2][0]), "+v"(xa[2][1]), "+v"(xa[3][0]), "+v"(xa[3][1]),
-                           "+v"(wb[0]), "+v"(wb[1]), "+v"(wb[2]), "+v"(wb[3]));
-            /* every output takes its hi product, then its lo product; the
-             * 16 hi MFMAs go first so that no MFMA waits on the one just
-             * issued */
+    for (int g = 0; g < LMG_GPW; g++) { bv[g] = __builtin_nanf(""); bi[g] = 0x7fffffff; }
+    if (wave < LMG_MMW) {
+        const bool v4 = N % 4 == 0;   /* rows of y 16-byte aligned */
+        const int total = np * nch;
+        i32x4 wv[2][LMG_UPW], xa[2][2][LMG_GPW];
+        auto read = [&](int sw, int sc, int sx, int s) {
+            /* rows of all fragments agree mod 16: one swizzle per operand */
+            const uint32_t q = (uint32_t)(l16 * 128 + 16 * ((4 * s + g4) ^ lmg_swz(l16, 8)));
+            const uint32_t qw = (uint32_t)(l16 * 16 * LMG_PPR + 16 * ((8 * sc + 4 * s + g4) ^ lmg_swz(l16, LMG_PPR)));
+            const uint32_t wb = ldsw + (uint32_t)(sw * MM_LMG_WB) + qw, xb = ldsx + (uint32_t)(sx * MM_LMG_XB) + q;
+#pragma unroll
+            for (int j = 0; j < LMG_UPW; j++)   /* a wave with fewer units repeats the last one, unused */
+                wv[s][j] = *(lmg_lds_cp)(wb + (uint32_t)(min(wu + 4 * j, MM_LMG_MU - 1) * 256 * LMG_PPR));
 #pragma unroll
             for (int h = 0; h < 2; h++)
 #pragma unroll
-                for (int g = 0; g < 4; g++)
+                for (int g = 0; g < LMG_GPW; g++) xa[s][h][g] = *(lmg_lds_cp)(xb + (uint32_t)((64 * h + 16 * (g0 + g)) * 128));
+        };
+        f32x4 acc[LMG_UPW][LMG_GPW];
+        auto zero = [&]() {
 #pragma unroll
-                    for (int j = 0; j < 4; j++)
+            for (int j = 0; j < LMG_UPW; j++)
+#pragma unroll
+                for (int g = 0; g < LMG_GPW; g++) acc[j][g] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+        };
+        auto mfma = [&](int s) {
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int g = 0; g < LMG_GPW; g++)
+#pragma unroll
+                    for (int j = 0; j < LMG_UPW; j++)
                         acc[j][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                            __builtin_bit_cast(lmg_bf16x8, xa[g][h]),
-                            __builtin_bit_cast(lmg_bf16x8, wb[j]), acc[j][g], 0, 0, 0);
-        }
-    }
-    /* C[token 16 g + 4 (l / 16) + i][column n0 + 64 wave + 16 j + l % 16] */
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int n = n0 + 64 * wave + 16 * j + (lane & 15);
-        if (n >= N) continue;
-#pragma unroll
-        for (int g = 0; g < 4; g++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int t = 16 * g + 4 * (lane >> 4) + i;
-                if (t < T) a.y[(size_t)t * N + n] = acc[j][g][i];
+                            __builtin_bit_cast(lmg_bf16x8, wv[s][j]),
+                            __builtin_bit_cast(lmg_bf16x8, xa[s][h][g]), acc[j][g], 0, 0, 0);
+        };
+        int sw = 0, sc = 0, sx = 0, c = 0, p = 0;   /* W slot, chunk within it, x slot; chunk, pass */
+        zero();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        read(0, 0, 0, 0);
+        for (int i = 0; i < total; i++) {
+            read(sw, sc, sx, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            mfma(0);
+            __builtin_amdgcn_sched_barrier(0);
+            /* this wave's reads of the slots are done before the barrier that
+             * frees them and makes the next chunk's loads visible */
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            const bool last = ++c == nch;
+            sx = sx + 1 == MM_LMG_NSX ? 0 : sx + 1;
+            if (++sc == MM_LMG_WC || last) {
+                sc = 0;
+                sw = sw + 1 == MM_LMG_NSW ? 0 : sw + 1;
             }
+            if (i + 1 < total) {
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                read(sw, sc, sx, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            mfma(1);
+            __builtin_amdgcn_sched_barrier(0);
+            if (!last) continue;
+            /* C[column 16 u + 4 (l / 16) + i][token 16 g + l % 16] */
+            const int u0 = first(p), un_p = first(p + 1) - u0;
+#pragma unroll
+            for (int j = 0; j < LMG_UPW; j++) {
+                const int u = wu + 4 * j, n = 16 * (u0 + u) + 4 * g4;
+                if (u >= un_p) continue;
+#pragma unroll
+                for (int g = 0; g < LMG_GPW; g++) {
+                    const int t = 16 * (g0 + g) + l16;
+                    if (t >= T || n >= N) continue;
+                    float *y = a.y + (size_t)t * N + n;
+                    if (v4) __builtin_nontemporal_store(acc[j][g], (f32x4 *)y);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        if (n + k >= N) continue;
+                        if (!v4) y[k] = acc[j][g][k];
+                        if (am_better(acc[j][g][k], n + k, bv[g], bi[g])) { bv[g] = acc[j][g][k]; bi[g] = n + k; }
+                    }
+                }
+            }
+            c = 0;
+            p++;
+            zero();
+        }
+#pragma unroll
+        for (int off = 16; off < MM_WAVE; off <<= 1)
+#pragma unroll
+            for (int g = 0; g < LMG_GPW; g++) {
+                const float ov = __shfl_xor(bv[g], off, MM_WAVE);
+                const int oi = __shfl_xor(bi[g], off, MM_WAVE);
+                if (am_better(ov, oi, bv[g], bi[g])) { bv[g] = ov; bi[g] = oi; }
+            }
+    }
+    /* the waves' bests meet in the (drained) ring's LDS */
+    __syncthreads();
+    float *sv = (float *)lds;             /* [4][64] */
+    int *si = (int *)(lds + 4 * 64 * 4);
+    if (wave < LMG_MMW && g4 == 0)
+#pragma unroll
+        for (int g = 0; g < LMG_GPW; g++) {
+            sv[wu * 64 + 16 * (g0 + g) + l16] = bv[g];
+            si[wu * 64 + 16 * (g0 + g) + l16] = bi[g];
+        }
+    __syncthreads();
+    if (tid < T) {
+        float v = sv[tid];
+        int ix = si[tid];
+        for (int w = 1; w < 4; w++)
+            if (am_better(sv[w * 64 + tid], si[w * 64 + tid], v, ix)) { v = sv[w * 64 + tid]; ix = si[w * 64 + tid]; }
+        a.part_v[(size_t)tid * gridDim.x + blockIdx.x] = v;
+        a.part_i[(size_t)tid * gridDim.x + blockIdx.x] = ix;
     }
 }
