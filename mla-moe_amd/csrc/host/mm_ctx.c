@@ -175,9 +175,10 @@ int mm_ctx_create(int device, mm_ctx **out) {
             goto fail;
         }
     }
-    /* MLAMOE_I8_TILED_MIN_T overrides the token count from which the int8
-     * path switches to the tiled GEMM (for measuring the crossover). */
-    c->i8_tiled_min_t = 256;
+    /* MLAMOE_I8_TILED_MIN_T sets the token count from which the int8 path
+     * takes the tiled GEMMs, in place of the rule in forward_int8 (for
+     * measuring the crossover). */
+    c->i8_tiled_min_t = -1;
     const char *ev = getenv("MLAMOE_I8_TILED_MIN_T");
     if (ev && *ev) c->i8_tiled_min_t = atoi(ev);
     /* MLAMOE_MLA_PART_MAX (bytes) overrides the cap on the attention chunk

@@ -141,7 +141,7 @@ struct mm_ctx {
     mm_mla_front_config front;  /* rope_inv_freq points at front_inv (device) */
     float *front_inv;           /* [qk_rope_head_dim / 2] device RoPE table */
 
-    int i8_tiled_min_t;         /* token count from which the tiled int8 GEMM is used */
+    int i8_tiled_min_t;         /* token count from which the tiled int8 GEMM is used (-1: by rule) */
     size_t mla_part_max;        /* attention chunk partials per launch (bytes) */
     int mla_expand_min;         /* rows of one sequence from which a step's attention is
                                    expanded (MLAMOE_MLA_EXPAND_MIN overrides) */

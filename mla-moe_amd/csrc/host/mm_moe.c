@@ -899,7 +899,8 @@ static int forward_int8(mm_ctx *c, const mm_moe_layer *L, int T, const float *xn
     /* decode-shaped GEMMs stage a 16-row A tile (16 * K bytes) and a row list
      * (T ints) in LDS; shapes beyond 64 KB of it take the tiled GEMMs */
     const size_t lds_dec = 16 * (H > (I > S ? I : S) ? H : (I > S ? I : S)) + 4 * (size_t)T;
-    const int tiled = T >= c->i8_tiled_min_t || lds_dec > 65536;
+    const int tiled = lds_dec > 65536 || (c->i8_tiled_min_t >= 0 ? T >= c->i8_tiled_min_t
+                                                                 : T >= MM_I8_TILED_T || R >= MM_I8_TILED_ROWS * E);
     /* per-expert row lists only for the tiled path; the decode-shaped GEMMs
      * build theirs from the routing */
     ra.cnt = tiled ? c->moe_cnt : NULL;

@@ -306,6 +306,17 @@ typedef struct {
 #define MM_I8S_RT 4                /* row-tile blocks per shared-expert column group */
 #define MM_I8S_XCD 8               /* blocks are dealt to XCDs round robin */
 
+/* Tiled GEMMs from MM_I8_TILED_T tokens on, or from MM_I8_TILED_ROWS rows per
+ * expert on average.  A decode-shaped block streams its expert's weights once
+ * per 16 rows, so its time doubles soon after the experts' row counts pass 16;
+ * a tile reads them once per 128 rows but costs more to fill.  Whole layer
+ * (DeepSeek-V2-Lite: 64 experts, 6 per token, even routing), decode-shaped ->
+ * tiled: 96 tokens (9 rows) 142 -> 166 us, 112 tokens 152 -> 168, 160 tokens
+ * (15 rows) 210 -> 169, 255 tokens 281 -> 177; Zipf-skewed routing crosses
+ * below 56 tokens, which the host cannot know (it does not see the routing). */
+#define MM_I8_TILED_T 256
+#define MM_I8_TILED_ROWS 12
+
 /* Grouped int8 GEMM for prefill sizes (mm_i8_gemm_bt, gemm_i8.hip): block
  * tiles of 128 rows x 16 B fragments over the routed experts' row lists (or
  * all T rows for the shared expert), a persistent grid of two blocks per CU. */
