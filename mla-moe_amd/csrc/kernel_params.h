@@ -89,7 +89,7 @@ typedef struct {
 #endif
 #define MM_BF16_MM_T_CHUNK 2048   /* rows of one pass (its workspace: ~180 KB per row) */
 #define MM_BF16_MM_GRID 256       /* persistent grid: one block per CU */
-#define MM_BF16_MM_THREADS 320    /* four multiplying waves and one loading activations */
+#define MM_BF16_MM_THREADS 512    /* four multiplying waves, two loading weights, two activations */
 /* The load rings of 16-, 32- and 64-row tiles (dynamic LDS): NSW stages of KB
  * values of K of 128 weight rows, NSA of the three planes of the rows */
 #ifndef MM_BF16_MM_KB

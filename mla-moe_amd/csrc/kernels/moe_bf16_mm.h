@@ -20,10 +20,9 @@
  * one contiguous run: no row lists inside the GEMM's load loop.
  *
  * Measured on a DeepSeek-V2-Lite layer, GEMV stages -> these kernels: 64
- * tokens 1430 -> 248 us, 515 tokens 11,440 -> 446 us.  At 64 tokens the weight
+ * tokens 1430 -> 245 us, 515 tokens 11,440 -> 431 us.  At 64 tokens the weight
  * stream bounds them: gate/up 761 MB in 144 us (5.3 TB/s), down 381 MB in 78
- * us (4.9 TB/s); with more rows per expert LDS reads and MFMAs share the time
- * (272 and 145 us at 515 tokens).
+ * us (4.9 TB/s); with more rows per expert LDS reads and MFMAs share the time.
  */
 #pragma once
 #include "common.h"
@@ -107,11 +106,14 @@ extern "C" __global__ __launch_bounds__(256) void mm_bf16_rows(mm_bf16_rows_args
  * Both operands go global -> LDS by direct loads of whole 128-byte lines, in
  * two rings: weights NSW stages, activation planes NSA.  The grid is
  * persistent, one block per CU, and the rings run across tile boundaries, so
- * the weight stream does not pause at a tile's start or end.  Four waves
- * multiply and load the weights; a fifth loads the planes: a wave's vector
+ * the weight stream does not pause at a tile's start or end.  Four waves only
+ * read LDS and multiply, two load weights and two load planes: a wave's vector
  * memory operations complete in order, so a wave loading both could not wait
  * for planes (an L2 hit, needed soon) without waiting for weights issued
- * before them (from HBM, wanted as far ahead as LDS allows).  LDS rows are
+ * before them (from HBM, wanted as far ahead as LDS allows), nor a multiplying
+ * wave load without waiting for its stores.  With the weights loaded by the
+ * multiplying waves and one wave for the planes, 515 tokens took 451 us; the
+ * loading waves give 446, the reads between the MFMAs 431.  LDS rows are
  * KB * 2 bytes of 16-byte pieces, piece p of row r in slot p ^ swz(r): 16
  * rows at one piece fall on distinct bank groups.  BM 16 or 32: each
  * multiplying wave owns all rows and a quarter of the weight rows; BM 64: a
@@ -120,7 +122,7 @@ extern "C" __global__ __launch_bounds__(256) void mm_bf16_rows(mm_bf16_rows_args
  * past Kd) are out of the buffer's range: no memory is read and zeros are
  * staged.
  *
- * The operands of the next 32-wide K step are read from LDS during the
+ * The operands of the next 32-wide K step are read from LDS between the
  * current step's MFMAs (plain loads, which the compiler counts), the first
  * step of the next chunk included: the wait for that chunk and the block's
  * barrier come before a chunk's last MFMAs.
@@ -132,13 +134,17 @@ extern "C" __global__ __launch_bounds__(256) void mm_bf16_rows(mm_bf16_rows_args
 #define GRP_OOB 0xFFFFFFF0u           /* past every buffer range */
 #define GRP_FLUSH 256
 #define GRP_MMW 4                     /* multiplying waves */
+#define GRP_WLD 2                     /* weight-loading waves */
+#define GRP_ALD 2                     /* plane-loading waves */
+static_assert(MM_BF16_MM_THREADS == (GRP_MMW + GRP_WLD + GRP_ALD) * MM_WAVE, "threads known to the host");
 
 template <int BM> struct shape {
     static constexpr int KB = MM_BF16_MM_KB(BM);
     static constexpr int ROWB = 2 * KB;                /* LDS bytes per row */
     static constexpr int RPI = 1024 / ROWB;            /* rows per load instruction */
-    static constexpr int W_LPW = GRP_NB / RPI / GRP_MMW;       /* weight loads per wave per chunk */
-    static constexpr int A_INS = 3 * BM / RPI;         /* plane loads per chunk */
+    static constexpr int W_LPW = GRP_NB / RPI / GRP_WLD;       /* loads per weight-loading wave per chunk */
+    static constexpr int AP = BM / RPI / GRP_ALD;      /* loads per plane-loading wave, plane and chunk */
+    static constexpr int A_LPW = 3 * AP;
     static constexpr int W_BYTES = GRP_NB * ROWB, A_BYTES = 3 * BM * ROWB;
     static constexpr int NSW = MM_BF16_MM_NSW(BM), NSA = MM_BF16_MM_NSA(BM);
     static constexpr int WN = BM == 64 ? 2 : 4;        /* waves over the weight rows */
@@ -146,7 +152,7 @@ template <int BM> struct shape {
     static constexpr int WT = GRP_NB / 16 / WN;            /* 16-column weight tiles per wave */
     static constexpr int KS = KB / 32;                 /* MFMA steps per chunk */
     static_assert(NSW * W_BYTES + NSA * A_BYTES == MM_BF16_MM_LDS(BM), "ring sizes known to the host");
-    static_assert(W_LPW * (NSW - 2) < 64 && A_INS * (NSA - 2) < 64 && KS % 2 == 0 && GRP_FLUSH % KB == 0, "");
+    static_assert(W_LPW * (NSW - 2) < 64 && A_LPW * (NSA - 2) < 64 && KS % 2 == 0 && GRP_FLUSH % KB == 0, "");
     static __device__ int swz(int r) { return KB == 64 ? (r >> 1) & 7 : r & 15; }
 };
 
@@ -162,6 +168,8 @@ struct grp_tile {
     int si, e, slab, m0, M;        /* segment, expert, column slab, first row, the expert's rows */
     int row0;                      /* sorted position of the expert's first row */
 };
+
+template <int V> struct const_int { static constexpr int v = V; };
 
 template <int BM, bool GU>
 __device__ __forceinline__ grp_tile grp_decode(const mm_bf16_mm_args &a, const grp_shared &sh, int n0, int t) {
@@ -252,9 +260,9 @@ __device__ __forceinline__ void grp_run(const mm_bf16_mm_args &a) {
 
     /* ---- loads ----
      * a load instruction covers RPI LDS rows; lane l carries row + l / LPR,
-     * slot l % LPR, i.e. K piece slot ^ swz(row).  Weight load W_LPW wave + u
-     * covers the weight rows from RPI times it; plane load i (the loading
-     * wave's) plane i / (BM / RPI), rows from RPI (i % (BM / RPI)). */
+     * slot l % LPR, i.e. K piece slot ^ swz(row).  Load u of loading wave lw
+     * covers the rows from RPI (W_LPW lw + u) of the weights, or from RPI (AP
+     * lw + u) of each plane. */
     constexpr int RPI = sp::RPI, LPR = MM_WAVE / RPI, KB = sp::KB;
     const uint32_t ldsw = lds_addr(lds), ldsa = ldsw + sp::NSW * sp::W_BYTES;
     auto piece = [&](int r) { return 8 * ((lane % LPR) ^ sp::swz(r)); };   /* first K value */
@@ -272,10 +280,35 @@ __device__ __forceinline__ void grp_run(const mm_bf16_mm_args &a) {
         return true;
     };
 
-    if (wave == GRP_MMW) {   /* the planes' wave */
+    /* A loading wave's ring of NS stages, LPW loads each: NS - 1 chunks are
+     * out before the first barrier, and each chunk's barrier shows that the
+     * next one has landed (only those of the NS - 2 chunks after it are out)
+     * and that every read of the chunk is done, whose slot the issues after
+     * the barrier take. */
+    auto load_ring = [&](auto ns, auto lpw, auto &issue) {
+        constexpr int NS = decltype(ns)::v, OUT = decltype(lpw)::v * (NS - 2);
+#pragma unroll 1
+        for (int s = 0; s < NS - 1; s++) issue(s);
+        VMCNT_WAIT(OUT);
+        __builtin_amdgcn_s_barrier();
+        int slot = NS - 1;
+        for (; ct < len; ct += nbx) {
+            const int nch = (a.seg[tile_at(ct).si].Kd + KB - 1) / KB;
+            for (int cc = 0; cc < nch; cc++) {
+                issue(slot);
+                slot = slot + 1 == NS ? 0 : slot + 1;
+                VMCNT_WAIT(OUT);
+                __builtin_amdgcn_s_barrier();
+            }
+        }
+        VMCNT_WAIT(0);
+    };
+    if (wave >= GRP_MMW + GRP_WLD) {   /* a planes' wave */
+        const int lw = wave - GRP_MMW - GRP_WLD;
         rsrc_t ar[3];
-        constexpr int AP = sp::A_INS / 3;              /* loads per plane */
+        constexpr int AP = sp::AP;
         uint32_t ao[AP];
+        auto row_of = [&](int u) { return RPI * (AP * lw + u) + lane / LPR; };
         auto set_issue = [&](const grp_tile &id) {
             const mm_bf16_mm_seg &g = a.seg[id.si];
             kd = g.Kd;
@@ -287,65 +320,57 @@ __device__ __forceinline__ void grp_run(const mm_bf16_mm_args &a) {
                                  (uint32_t)rows * (uint32_t)kd * 2u);
 #pragma unroll
             for (int u = 0; u < AP; u++) {
-                const int R = RPI * u + lane / LPR;
+                const int R = row_of(u);
                 ao[u] = R < rows ? ((uint32_t)R * (uint32_t)kd + (uint32_t)piece(R)) * 2u : GRP_OOB;
             }
         };
         auto issue = [&](int slot) {
-            const uint32_t sb = ldsa + (uint32_t)(slot * sp::A_BYTES);
+            const uint32_t sb = ldsa + (uint32_t)(slot * sp::A_BYTES + AP * lw * 1024);
             const int k0 = ic * KB;
 #pragma unroll
             for (int u = 0; u < AP; u++) {
-                const uint32_t o = ao[u] != GRP_OOB && k0 + piece(RPI * u + lane / LPR) < kd ? ao[u] + (uint32_t)(2 * k0) : GRP_OOB;
+                const uint32_t o = ao[u] != GRP_OOB && k0 + piece(row_of(u)) < kd ? ao[u] + (uint32_t)(2 * k0) : GRP_OOB;
 #pragma unroll
-                for (int q = 0; q < 3; q++) lds_dma16_buf(o, ar[q], sb + (uint32_t)((q * AP + u) * 1024));
+                for (int q = 0; q < 3; q++) lds_dma16_buf(o, ar[q], sb + (uint32_t)((q * (BM / RPI) + u) * 1024));
             }
             if (advance()) set_issue(tile_at(it));
         };
         set_issue(tile_at(it));
-#pragma unroll 1
-        for (int s = 0; s < sp::NSA - 1; s++) issue(s);
-        VMCNT_WAIT(sp::A_INS * (sp::NSA - 2));
-        __builtin_amdgcn_s_barrier();
-        int slot = sp::NSA - 1;
-        for (; ct < len; ct += nbx) {
-            const int nch = (a.seg[tile_at(ct).si].Kd + KB - 1) / KB;
-            for (int cc = 0; cc < nch; cc++) {   /* one barrier per chunk, as the multiplying waves */
-                issue(slot);
-                slot = slot + 1 == sp::NSA ? 0 : slot + 1;
-                VMCNT_WAIT(sp::A_INS * (sp::NSA - 2));
-                __builtin_amdgcn_s_barrier();
-            }
-        }
-        VMCNT_WAIT(0);
+        load_ring(const_int<sp::NSA>(), const_int<sp::A_LPW>(), issue);
         return;
     }
 
-    rsrc_t wr[GU ? 2 : 1];
-    uint32_t wo[sp::W_LPW];
-    auto wload_row = [&](int u) { return RPI * (sp::W_LPW * wave + u) + lane / LPR; };
-    auto wup = [&](int u) { return GU && RPI * (sp::W_LPW * wave + u) >= GRP_NB / 2; };   /* uniform */
-    auto set_issue = [&](const grp_tile &id) {
-        const mm_bf16_mm_seg &g = a.seg[id.si];
-        kd = g.Kd;
-        inch = (kd + KB - 1) / KB;
-        wr[0] = raw_rsrc(g.w0 + (size_t)id.e * g.wstride, (uint32_t)g.N * (uint32_t)kd * 2u);
-        if (GU) wr[GU ? 1 : 0] = raw_rsrc(g.w1 + (size_t)id.e * g.wstride, (uint32_t)g.N * (uint32_t)kd * 2u);
+    if (wave >= GRP_MMW) {   /* a weights' wave */
+        const int lw = wave - GRP_MMW;
+        rsrc_t wr[GU ? 2 : 1];
+        uint32_t wo[sp::W_LPW];
+        auto row_of = [&](int u) { return RPI * (sp::W_LPW * lw + u) + lane / LPR; };
+        auto up = [&](int u) { return GU && RPI * (sp::W_LPW * lw + u) >= GRP_NB / 2; };   /* uniform */
+        auto set_issue = [&](const grp_tile &id) {
+            const mm_bf16_mm_seg &g = a.seg[id.si];
+            kd = g.Kd;
+            inch = (kd + KB - 1) / KB;
+            wr[0] = raw_rsrc(g.w0 + (size_t)id.e * g.wstride, (uint32_t)g.N * (uint32_t)kd * 2u);
+            if (GU) wr[GU ? 1 : 0] = raw_rsrc(g.w1 + (size_t)id.e * g.wstride, (uint32_t)g.N * (uint32_t)kd * 2u);
 #pragma unroll
-        for (int u = 0; u < sp::W_LPW; u++) {
-            const int R = wload_row(u), col = id.slab * CPT + (GU ? R & 63 : R);
-            wo[u] = col < g.N ? ((uint32_t)col * (uint32_t)kd + (uint32_t)piece(R)) * 2u : GRP_OOB;
-        }
-    };
-    auto issue = [&](int slot) {
-        const uint32_t sb = ldsw + (uint32_t)(slot * sp::W_BYTES + sp::W_LPW * wave * 1024);
-        const int k0 = ic * KB;
+            for (int u = 0; u < sp::W_LPW; u++) {
+                const int R = row_of(u), col = id.slab * CPT + (GU ? R & 63 : R);
+                wo[u] = col < g.N ? ((uint32_t)col * (uint32_t)kd + (uint32_t)piece(R)) * 2u : GRP_OOB;
+            }
+        };
+        auto issue = [&](int slot) {
+            const uint32_t sb = ldsw + (uint32_t)(slot * sp::W_BYTES + sp::W_LPW * lw * 1024);
+            const int k0 = ic * KB;
 #pragma unroll
-        for (int u = 0; u < sp::W_LPW; u++)
-            lds_dma16_buf_nt(wo[u] != GRP_OOB && k0 + piece(wload_row(u)) < kd ? wo[u] + (uint32_t)(2 * k0) : GRP_OOB,
-                             wup(u) ? wr[GU ? 1 : 0] : wr[0], sb + (uint32_t)(u * 1024));
-        if (advance()) set_issue(tile_at(it));
-    };
+            for (int u = 0; u < sp::W_LPW; u++)
+                lds_dma16_buf_nt(wo[u] != GRP_OOB && k0 + piece(row_of(u)) < kd ? wo[u] + (uint32_t)(2 * k0) : GRP_OOB,
+                                 up(u) ? wr[GU ? 1 : 0] : wr[0], sb + (uint32_t)(u * 1024));
+            if (advance()) set_issue(tile_at(it));
+        };
+        set_issue(tile_at(it));
+        load_ring(const_int<sp::NSW>(), const_int<sp::W_LPW>(), issue);
+        return;
+    }
 
     /* ---- operand reads ----
      * weight tile j of this wave: LDS rows wrow(j) + l % 16; row tile t: plane
@@ -387,6 +412,13 @@ __device__ __forceinline__ void grp_run(const mm_bf16_mm_args &a) {
                     c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, rw[s & 1][j]),
                                                                 __builtin_bit_cast(bf16x8, rx[s & 1][t][q]), c, 0, 0, 0);
                 }
+        /* the next step's reads between the MFMAs */
+        constexpr int RD = WT + 3 * TT, MF = 3 * TT * WT, PER = MF / RD > 0 ? MF / RD : 1;
+#pragma unroll
+        for (int i = 0; i < RD; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, PER, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
     };
     auto flush = [&]() {
 #pragma unroll
@@ -432,18 +464,9 @@ __device__ __forceinline__ void grp_run(const mm_bf16_mm_args &a) {
         }
     };
 
-    set_issue(tile_at(it));
-#pragma unroll 1
-    for (int s = 0; s < sp::NSW - 1; s++) issue(s);
     grp_tile cur = tile_at(ct);
     int nch = (a.seg[cur.si].Kd + KB - 1) / KB, cc = 0, sw = 0, sa = 0;
     zero();
-    /* a chunk's loads of this wave have landed once only those of the NSW - 2
-     * chunks after it are out (stores of a tile's end in between make this
-     * stricter).  The barrier before chunk n + 1: every wave's loads of it,
-     * and every wave's reads of chunk n (waited for before the barrier), whose
-     * slot the issues after the barrier take. */
-    VMCNT_WAIT(sp::W_LPW * (sp::NSW - 2));
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     read(0, 0, 0);
@@ -451,17 +474,14 @@ __device__ __forceinline__ void grp_run(const mm_bf16_mm_args &a) {
         const int nw = sw + 1 == sp::NSW ? 0 : sw + 1, na = sa + 1 == sp::NSA ? 0 : sa + 1;
 #pragma unroll
         for (int s = 0; s < KS; s++) {
-            if (s == 0) issue(sw == 0 ? sp::NSW - 1 : sw - 1);
             if (s + 1 < KS) {
                 read(sw, sa, s + 1);
             } else {
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                VMCNT_WAIT(sp::W_LPW * (sp::NSW - 2));
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
                 read(nw, na, 0);
             }
-            __builtin_amdgcn_sched_barrier(0);
             mfma(s);
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -479,11 +499,10 @@ __device__ __forceinline__ void grp_run(const mm_bf16_mm_args &a) {
             flush();
         }
     }
-    VMCNT_WAIT(0);
 }
 
 #define GRP_KERNEL(name, BM, GU)                                                            \
-    extern "C" __global__ __launch_bounds__((GRP_MMW + 1) * MM_WAVE, 1) void name(mm_bf16_mm_args a) { grp_run<BM, GU>(a); }
+    extern "C" __global__ __launch_bounds__(MM_BF16_MM_THREADS, 1) void name(mm_bf16_mm_args a) { grp_run<BM, GU>(a); }
 GRP_KERNEL(mm_bf16_gu_16, 16, true)
 GRP_KERNEL(mm_bf16_gu_32, 32, true)
 GRP_KERNEL(mm_bf16_gu_64, 64, true)
