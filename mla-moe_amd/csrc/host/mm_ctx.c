@@ -61,6 +61,7 @@ static const struct {
     [K_I8_COMBINE_NORM] = {"mm_i8_combine_norm", MOD_MOE_I8},
     [K_PACK_I8] = {"mm_pack_i8", MOD_MOE_I8},
     [K_I8_BT_GU] = {"mm_i8_gemm_gu", MOD_GEMM_I8},
+    [K_I8_BT_GU_EX] = {"mm_i8_gemm_gu_ex", MOD_GEMM_I8},
     [K_I8_BT_DN] = {"mm_i8_gemm_dn", MOD_GEMM_I8},
     [K_I8_BT_GU_DBG] = {"mm_i8_gemm_gu_dbg", MOD_GEMM_I8},
     [K_I8_BT_DN_DBG] = {"mm_i8_gemm_dn_dbg", MOD_GEMM_I8},

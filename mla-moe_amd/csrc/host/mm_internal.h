@@ -38,6 +38,7 @@ typedef enum {
     K_I8_COMBINE_NORM,
     K_PACK_I8,
     K_I8_BT_GU,
+    K_I8_BT_GU_EX,
     K_I8_BT_DN,
     K_I8_BT_GU_DBG,
     K_I8_BT_DN_DBG,

@@ -821,7 +821,7 @@ static int launch_tiled(mm_ctx *c, const mm_i8_tiled_args *ta, const mm_i8_tiled
     ba.seg[0] = *ta;
     if (ts) ba.seg[1] = *ts;
     ba.nseg = ts ? 2 : 1;
-    const mm_kernel_id k = ta->gu ? (ta->dbg_acc ? K_I8_BT_GU_DBG : K_I8_BT_GU)
+    const mm_kernel_id k = ta->gu ? (ta->dbg_acc ? K_I8_BT_GU_DBG : ta->gu == 2 ? K_I8_BT_GU_EX : K_I8_BT_GU)
                                   : (ta->dbg_acc ? K_I8_BT_DN_DBG : K_I8_BT_DN);
     return mm_launch(c, k, MM_I8B_GRID, 1, 1, 256, 0, &ba);
 }
@@ -901,6 +901,9 @@ static int forward_int8(mm_ctx *c, const mm_moe_layer *L, int T, const float *xn
     const size_t lds_dec = 16 * (H > (I > S ? I : S) ? H : (I > S ? I : S)) + 4 * (size_t)T;
     const int tiled = lds_dec > 65536 || (c->i8_tiled_min_t >= 0 ? T >= c->i8_tiled_min_t
                                                                  : T >= MM_I8_TILED_T || R >= MM_I8_TILED_ROWS * E);
+    /* which SwiGLU: a call that the rows per expert alone made tiled has the
+     * decode-shaped GEMM's */
+    const int gu = lds_dec <= 65536 && c->i8_tiled_min_t < 0 && T < MM_I8_TILED_T ? 2 : 1;
     /* per-expert row lists only for the tiled path; the decode-shaped GEMMs
      * build theirs from the routing */
     ra.cnt = tiled ? c->moe_cnt : NULL;
@@ -947,9 +950,9 @@ static int forward_int8(mm_ctx *c, const mm_moe_layer *L, int T, const float *xn
         /* routed experts, then the shared expert as one dense GEMM */
         mm_i8_tiled_args ta = {L->i8.gu, 2 * I * H, L->i8.s_g, L->i8.s_u, (int)I, c->moe_cnt,
                                rows, qx, sx, 0, h, dbg ? dbg->acc_gu : NULL, T, (int)K,
-                               (int)E, (int)I, (int)H, 1, (int)R};
+                               (int)E, (int)I, (int)H, gu, (int)R};
         mm_i8_tiled_args ts = {L->i8.sgu, 0, L->i8.ss_g, L->i8.ss_u, 0, NULL, NULL, qx, sx, 0,
-                               hs, NULL, T, (int)K, 1, (int)S, (int)H, 1, T};
+                               hs, NULL, T, (int)K, 1, (int)S, (int)H, gu, T};
         FAIL_ROUTED(launch_tiled(c, &ta, S ? &ts : NULL));
     } else {
         /* shared-expert blocks (row-tile waves), then every routed unit */

@@ -236,7 +236,7 @@ struct bt_xcd_list {
     __device__ int operator()(int t) const { return t < len0 ? lo0 + t : lo1 + (t - len0); }
 };
 
-template <bool GU, bool DBG>
+template <bool GU, bool DBG, bool EX = false>
 __device__ __forceinline__ void bt_run(const mm_i8_bt_args &a, int8_t *lds, float *ep, bt_shared &sh,
                                        const bt_xcd_list &xl, int t, int t_step) {
     const int t_end = xl.len;
@@ -568,9 +568,11 @@ __device__ __forceinline__ void bt_run(const mm_i8_bt_args &a, int8_t *lds, floa
                         if (GU) {
                             const f32x4 c1 = *(const f32x4 *)(&sh.cs[buf][128 + cl]);
 #pragma unroll
-                            for (int i = 0; i < 4; i++)
-                                v[i] = silu_mul_fast(((float)acc[ri][0][4 * gq + i] * sa) * c0[i],
-                                                     ((float)acc[ri][1][4 * gq + i] * sa) * c1[i]);
+                            for (int i = 0; i < 4; i++) {
+                                const float gv = ((float)acc[ri][0][4 * gq + i] * sa) * c0[i];
+                                const float uv = ((float)acc[ri][1][4 * gq + i] * sa) * c1[i];
+                                v[i] = EX || (DBG && g.gu == 2) ? silu_mul(gv, uv) : silu_mul_fast(gv, uv);
+                            }
                             if (DBG && dbg) {
                                 const int rid = sh.rid[buf][32 * ri + l32], col = slab_c0 + cl;
                                 if (rid >= 0 && col < N) {
@@ -630,7 +632,7 @@ __device__ __forceinline__ void bt_run(const mm_i8_bt_args &a, int8_t *lds, floa
  * those tiles in turn, so the blocks of one XCD work on neighbouring tiles at
  * the same time: row groups of the same expert and slab, whose weights then
  * come from HBM once and from that XCD's L2 for the others. */
-template <bool GU, bool DBG>
+template <bool GU, bool DBG, bool EX = false>
 __device__ __forceinline__ void bt_kernel(const mm_i8_bt_args &a) {
     __shared__ __attribute__((aligned(1024))) int8_t lds[BT_NSA * BT_A_BYTES];
     __shared__ __attribute__((aligned(16))) float ep[4 * 32 * BT_EP_LD];
@@ -674,13 +676,17 @@ __device__ __forceinline__ void bt_kernel(const mm_i8_bt_args &a) {
     xl.lo1 = n0 + n1 * xcd / MM_I8S_XCD;
     xl.len = xl.len0 + n0 + n1 * (xcd + 1) / MM_I8S_XCD - xl.lo1;
     if (j >= xl.len) return;
-    bt_run<GU, DBG>(a, lds, ep, sh, xl, j, nbx);
+    bt_run<GU, DBG, EX>(a, lds, ep, sh, xl, j, nbx);
 }
 
 /* One kernel per epilogue form, so that each holds only its own code:
- * gate/up (SwiGLU, segments' gu = 1) and down (plain dequantisation). */
+ * gate/up (SwiGLU, segments' gu = 1; _ex: gu = 2) and down (plain
+ * dequantisation). */
 extern "C" __global__ __launch_bounds__(256, 2) void mm_i8_gemm_gu(mm_i8_bt_args a) {
     bt_kernel<true, false>(a);
+}
+extern "C" __global__ __launch_bounds__(256, 2) void mm_i8_gemm_gu_ex(mm_i8_bt_args a) {
+    bt_kernel<true, false, true>(a);
 }
 extern "C" __global__ __launch_bounds__(256, 2) void mm_i8_gemm_dn(mm_i8_bt_args a) {
     bt_kernel<false, false>(a);
