@@ -169,14 +169,17 @@ static int gemm_bf16_rows(mm_ctx *c, float *y, const uint16_t *xh, const uint16_
     /* block tile columns: the widest of 128, 64, 32 that still gives 192
      * tiles (most of the 256 CUs), else 32 -- the projections of this path
      * have too few 128 x 128 tiles to fill the machine (measured per width) */
-    const size_t nby = ((size_t)T + MM_GB_BM - 1) / MM_GB_BM;
+    int span = MM_GB_BM;   /* rows (or columns) of a tile, by their bytes */
+    while ((size_t)span * (size_t)kp * 2 > MM_GB_SPAN) span /= 2;
+    const size_t nby = ((size_t)T + span - 1) / span;
     int bn = 32;
     for (int cw = 128; cw >= 64; cw /= 2)
         if ((((size_t)d_out + cw - 1) / cw + ((size_t)d1 + cw - 1) / cw) * nby >= 192) {
             bn = cw;
             break;
         }
-    const size_t nb0 = ((size_t)d_out + bn - 1) / bn, nbx = nb0 + ((size_t)d1 + bn - 1) / bn;
+    const int cols = bn < span ? bn : span;
+    const size_t nb0 = ((size_t)d_out + cols - 1) / cols, nbx = nb0 + ((size_t)d1 + cols - 1) / cols;
     /* the XCDs' rectangle of tiles: fewest rounds of an XCD's 32 CUs, then
      * fewest operand rows read into an XCD's L2 (x rows count once per plane) */
     size_t best = 0, blocks = 0;
@@ -189,7 +192,8 @@ static int gemm_bf16_rows(mm_ctx *c, float *y, const uint16_t *xh, const uint16_
         xr = r;
         blocks = 8 * pr * pc;
     }
-    mm_gemm_bf16_args a = {xh, xl, w, y, T, d_out, n_in, kp, split, acc, bn, (int)nb0, d1 ? w1 : NULL, y1, d1, xr};
+    mm_gemm_bf16_args a = {xh, xl, w, y, T, d_out, n_in, kp, split, acc, bn, (int)nb0, d1 ? w1 : NULL, y1, d1, xr,
+                           span, cols};
     const size_t lds = (size_t)MM_GB_NS(split, bn) * MM_GB_STAGE(split, bn);
     return mm_launch(c, K_GEMM_BF16, (unsigned)blocks, 1, 1, 512, lds, &a);
 }

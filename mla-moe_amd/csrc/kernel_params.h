@@ -512,8 +512,13 @@ typedef struct {
     float *y1;
     int d_out1;
     int xr;                  /* the 8 XCDs as xr x 8 / xr rectangles of tiles: 1, 2, 4 or 8 */
+    int rows, cols;          /* a tile's rows and columns in use: MM_GB_BM and bn, fewer where
+                                n_in is so long that they span 4 GB (MM_GB_SPAN) */
 } mm_gemm_bf16_args;
 #define MM_GB_BM 128
+/* Bytes of x (one plane) or of weights that a tile may span: its loads have
+ * 32-bit offsets, the last 16 of which stand for "past the range". */
+#define MM_GB_SPAN 0xFFFFFFF0u
 /* LDS ring of mm_gemm_bf16: bytes per stage (A planes of 128 rows, bn rows of
  * B, 128 B each) and stages */
 #define MM_GB_STAGE(split, bn) (((split) ? 32768 : 16384) + (bn) * 128)

@@ -73,7 +73,9 @@ extern "C" __global__ __launch_bounds__(256) void mm_cvt_bf16(mm_cvt_bf16_args a
  * at position l % 8 of that row's 128 B the 16 B piece (l % 8) ^ s(row), s(R)
  * = (R / 2) % 8.  The XOR swizzle makes the operand reads (16 rows, one piece
  * each) conflict-free.  Rows past T and columns past d_out, and weight pieces
- * past n_in, are out of the buffers' range: nothing is read, zeros staged. */
+ * past n_in, are out of the buffers' range: nothing is read, zeros staged.
+ * Offsets within a tile's rows are 32 bits: where 128 rows of n_in values pass
+ * 4 GB (2^24 values) the tile takes fewer of them, down to one. */
 __device__ __forceinline__ int gb_swz(int R) { return (R >> 1) & 7; }
 typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -94,8 +96,8 @@ __device__ __forceinline__ void gemm_block(const mm_gemm_bf16_args &a, uint8_t *
      * b % 8).  The XCDs split the tile grid into xr x 8 / xr rectangles, so
      * that an XCD's L2 takes in 1 / xr of x and xr / 8 of the weights (the host
      * chooses xr).  Column blocks from nb0 on are the second matrix's. */
-    const int nb1 = a.w1 ? (a.d_out1 + BN - 1) / BN : 0;
-    const int nbx = a.nb0 + nb1, nby = (a.T + GB_BM - 1) / GB_BM;
+    const int nb1 = a.w1 ? (a.d_out1 + a.cols - 1) / a.cols : 0;
+    const int nbx = a.nb0 + nb1, nby = (a.T + a.rows - 1) / a.rows;
     const int xcd = blockIdx.x % 8, loc = blockIdx.x / 8, xc = 8 / a.xr;
     const int pr = (nby + a.xr - 1) / a.xr, pc = (nbx + xc - 1) / xc;
     const int rb = xcd / xc * pr + loc % pr;
@@ -105,12 +107,13 @@ __device__ __forceinline__ void gemm_block(const mm_gemm_bf16_args &a, uint8_t *
     if (second) cb -= a.nb0;
     const uint16_t *w = second ? a.w1 : a.w;
     const int d_out = second ? a.d_out1 : a.d_out;
-    const int m0 = rb * GB_BM, n0 = cb * BN;
+    const int m0 = rb * a.rows, n0 = cb * a.cols;
+    const int mrows = min(a.T - m0, a.rows), ncols = min(d_out - n0, a.cols);
     const int K = a.n_in, KB = a.kp / GB_BK;
     const uint32_t lds0 = lds_addr(lds);
 
     if (wave >= 4) {   /* a loading wave: a quarter of each plane and of the weights */
-        const int lw = wave - 4, mrows = min(a.T - m0, GB_BM), ncols = min(d_out - n0, BN);
+        const int lw = wave - 4;
         rsrc_t rs[NP + 1];
 #pragma unroll
         for (int q = 0; q < NP; q++)
@@ -137,11 +140,11 @@ __device__ __forceinline__ void gemm_block(const mm_gemm_bf16_args &a, uint8_t *
             for (int u = 0; u < 4; u++)
 #pragma unroll
                 for (int q = 0; q < NP; q++)
-                    lds_dma16_buf(ao[u] != GB_OOB ? ao[u] + (uint32_t)(2 * k0) : GB_OOB, rs[q],
+                    lds_dma16_buf(ao[u] != GB_OOB ? ao[u] + 2u * (uint32_t)k0 : GB_OOB, rs[q],
                                   sb + (uint32_t)(q * GB_COPY + (4 * lw + u) * 1024));
 #pragma unroll
             for (int u = 0; u < WL; u++)
-                lds_dma16_buf(wo[u] != GB_OOB && k0 + wk[u] < K ? wo[u] + (uint32_t)(2 * k0) : GB_OOB, rs[NP],
+                lds_dma16_buf(wo[u] != GB_OOB && k0 + wk[u] < K ? wo[u] + 2u * (uint32_t)k0 : GB_OOB, rs[NP],
                               sb + (uint32_t)(BOFF + (WL * lw + u) * 1024));
         };
 #pragma unroll 1
@@ -271,17 +274,18 @@ __device__ __forceinline__ void gemm_block(const mm_gemm_bf16_args &a, uint8_t *
      * unconditionally) before any is added. */
     float *y = second ? a.y1 : a.y;
     const bool acc_old = a.accumulate && !second;
+    const int mend = m0 + mrows, nend = n0 + ncols;
 #pragma unroll
     for (int t = 0; t < 2; t++) {
         const int m = m0 + 64 * wm + 32 * t + c32;
-        float *row = y + (size_t)min(m, a.T - 1) * d_out;
+        float *row = y + (size_t)min(m, mend - 1) * d_out;
         if (acc_old) {   /* uniform */
             f32x16 prev[WT];
 #pragma unroll
             for (int j = 0; j < WT; j++)
 #pragma unroll
                 for (int i = 0; i < 16; i++)
-                    prev[j][i] = row[min(n0 + cw + 32 * j + 8 * (i >> 2) + 4 * hi + (i & 3), d_out - 1)];
+                    prev[j][i] = row[min(n0 + cw + 32 * j + 8 * (i >> 2) + 4 * hi + (i & 3), nend - 1)];
 #pragma unroll
             for (int j = 0; j < WT; j++) sum[t][j] = prev[j] + sum[t][j];
         }
@@ -290,14 +294,14 @@ __device__ __forceinline__ void gemm_block(const mm_gemm_bf16_args &a, uint8_t *
 #pragma unroll
             for (int g = 0; g < 4; g++) {
                 const int n = n0 + cw + 32 * j + 8 * g + 4 * hi;
-                if (m >= a.T || n >= d_out) continue;
-                if (n + 3 < d_out) {
+                if (m >= mend || n >= nend) continue;
+                if (n + 3 < nend) {
                     *(f32x4_a4 *)(row + n) = (f32x4){sum[t][j][4 * g], sum[t][j][4 * g + 1], sum[t][j][4 * g + 2],
                                                      sum[t][j][4 * g + 3]};
                 } else {
 #pragma unroll
                     for (int i = 0; i < 3; i++)
-                        if (n + i < d_out) row[n + i] = sum[t][j][4 * g + i];
+                        if (n + i < nend) row[n + i] = sum[t][j][4 * g + i];
                 }
             }
     }

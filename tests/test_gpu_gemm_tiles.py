@@ -77,3 +77,32 @@ def test_two_matrices(ctx, oracle, T):
     # the bf16 pair of an fp32 input is off by up to 2^-18 of it
     for got, want in ((q, qr), (rows, cr)):
         assert np.linalg.norm(got - want) < 2.0 ** -18 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("T,d,n", [
+    (128, 3, (1 << 24) + 72),       # 128 rows of x span 4 GB
+    (2, 33, (1 << 26) + 8)])        # 32 rows of the weights do
+def test_rows_past_32_bit_offsets(ctx, T, d, n):
+    """Inner sizes at which a tile's rows span more than its loads' 32-bit
+    offsets: the tile takes fewer rows, and no row is lost.  x and W hold
+    whole numbers in a few columns, the first and the last among them, and
+    zeros elsewhere."""
+    print(f"long rows T={T} d={d} n={n}", flush=True)
+    rng = np.random.default_rng(T + d)
+    at = np.unique(np.r_[0, n - 1, n // 2, rng.integers(0, n, 12)])
+    xs, ws = ints(rng, (T, at.size)), ints(rng, (d, at.size))
+
+    def sparse(rows, values, kind, dtype):
+        buf = ctx.empty((rows, n), dtype)
+        ctx.fill(buf, rows * n, kind, 1, 0.0)          # deviation 0
+        one = np.empty(1, dtype)
+        for (r, j), v in np.ndenumerate(values):
+            one[0] = v
+            mlamoe._check(mlamoe.lib().mm_h2d(ctx.h, C.c_void_p(buf.ptr + (r * n + int(at[j])) * one.itemsize),
+                                              one.ctypes.data, one.itemsize))
+        return buf
+    x = sparse(T, xs, mlamoe.MM_FILL_F32_NORMAL, np.float32)
+    w = sparse(d, synth.bf16_from_f32(ws), mlamoe.MM_FILL_BF16_NORMAL, np.uint16)
+    y = ctx.empty((T, d), np.float32)
+    ctx.matmul_dev(y, x, w, d, n, T, mlamoe.MM_MATMUL_X_BF16)
+    assert np.array_equal(y.download(), xs @ ws.T)
