@@ -537,10 +537,12 @@ static bf16_mm_plan bf16_mm_layout(const mm_moe_config *g, size_t T, int logits)
     return w;
 }
 
-/* Weight matrices and activation tiles are read through 32-bit buffer offsets. */
+/* Weight matrices and tiles of up to 64 activation rows (H, I or S values
+ * each) are read through 32-bit buffer offsets. */
 static int bf16_mm_ok(const mm_moe_config *g) {
     const size_t H = g->hidden_size, I = g->moe_inter_size, S = (size_t)g->n_shared_experts * I;
-    return I * H < 0x7FFF0000u && S * H < 0x7FFF0000u;
+    const size_t w = I > S ? I : S;
+    return w * H < 0x7FFF0000u && 64 * (w > H ? w : H) < 0x7FFF0000u;
 }
 
 /* One pass over T tokens: router logits, routing with per-expert row lists,

@@ -129,3 +129,24 @@ def test_large_and_infinite_activations(inf):
     fin = np.isfinite(want)
     assert np.allclose(out[fin], want[fin], rtol=1e-6, atol=0)
     assert np.array_equal(out[~fin], want[~fin])
+
+
+def test_rows_past_32_bit_offsets():
+    """An intermediate size at which 64 hidden rows span 4 GB: the call takes
+    the GEMV stages.  The experts' weights are zero but for a few rows."""
+    H, E, K, I, NS, T = 8, 1, 1, 1 << 25, 0, 64
+    r = np.random.default_rng(980)
+    at = np.unique(np.r_[0, I - 1, r.integers(0, I, 12)])
+    w = synth.moe_layer(980, H, E, 8, NS)
+    for k, shape in (("eg", (E, I, H)), ("eu", (E, I, H)), ("ed", (E, H, I))):
+        w[k] = np.zeros(shape, np.uint16)
+    w["eg"][0, at], w["eu"][0, at] = synth.normal_bf16(r, (at.size, H)), synth.normal_bf16(r, (at.size, H))
+    w["ed"][0][:, at] = synth.normal_bf16(r, (H, at.size))
+    x = synth.activations(981, T, H)
+    with mlamoe.Context(0) as ctx:
+        ctx.moe_init(H, E, NS, K, I)
+        ctx.moe_load_layer(0, w, mlamoe.MM_LOAD_BF16)
+        out, idx, wt, _ = ctx.moe_forward(0, x)
+    few = dict(eg=w["eg"][:, at], eu=w["eu"][:, at], ed=w["ed"][:, :, at])
+    ref = ref64(few, x, idx, wt, NS)
+    assert np.linalg.norm(out - ref) < TOL * np.linalg.norm(ref)
