@@ -30,18 +30,25 @@
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
 
-/* x = hi + mid + lo, each a bf16, exactly: truncations of 8 significant bits
- * each (a rounded hi could overflow to infinity).  Infinities and NaN stay
- * in hi alone, so that they propagate as in fp32. */
+/* x = hi + mid + lo, each a bf16 of x's sign, exactly: truncations of 8
+ * significant bits each (a rounded hi could overflow to infinity).  Where a
+ * part would end the sum it is taken one step nearer to zero, so that no
+ * part of a nonzero x is zero: an infinite weight then gives infinity in
+ * every product, as in fp32, and not infinity + infinity * 0 (parts below
+ * 2^-133, of values below 2^-117, are zero all the same).  An infinite x gives
+ * infinity times whatever the weight is. */
 __device__ __forceinline__ void split3(float x, uint16_t *hi, uint16_t *mid, uint16_t *lo) {
     const uint32_t u = __float_as_uint(x);
     const bool fin = (u & 0x7f800000u) != 0x7f800000u;
-    *hi = x != x ? (uint16_t)0x7fc0u : (uint16_t)(u >> 16);
-    const float r1 = fin ? x - __uint_as_float(u & 0xffff0000u) : 0.0f;
-    const uint32_t u1 = __float_as_uint(r1);
-    const float r2 = r1 - __uint_as_float(u1 & 0xffff0000u);
-    *mid = (uint16_t)(u1 >> 16);
-    *lo = (uint16_t)(__float_as_uint(r2) >> 16);
+    auto part = [](uint32_t v) { return (v >> 16) - ((v & 0xffffu) == 0 && (v << 1) != 0 ? 1u : 0u); };
+    const uint32_t h = part(u);
+    const float r1 = x - __uint_as_float(h << 16);
+    const uint32_t m = part(__float_as_uint(r1));
+    const float r2 = r1 - __uint_as_float(m << 16);
+    const uint16_t one = (uint16_t)(((u >> 16) & 0x8000u) | 0x3f80u);
+    *hi = fin ? (uint16_t)h : x != x ? (uint16_t)0x7fc0u : (uint16_t)(u >> 16);
+    *mid = fin ? (uint16_t)m : one;
+    *lo = fin ? (uint16_t)(__float_as_uint(r2) >> 16) : one;
 }
 
 /* ---- sorted rows ------------------------------------------------------------ */

@@ -131,6 +131,55 @@ def test_large_and_infinite_activations(inf):
     assert np.array_equal(out[~fin], want[~fin])
 
 
+@pytest.mark.parametrize("where", ["eg", "eu", "ed", "sg", "su", "sd"])
+def test_infinite_weights(where):
+    """Infinite weights against activations exact in bf16, in two bf16 parts
+    and in none: the infinities and NaN of 4 rows at a time (the GEMV, fp32
+    products), and its values elsewhere."""
+    H, E, K, I, NS, T = 64, 4, 2, 64, 1, 24
+    r = np.random.default_rng(973)
+    w = synth.moe_layer(974, H, E, I, NS)
+    v = w[where].reshape(-1, w[where].shape[-1])
+    v[r.integers(0, v.shape[0], 6), r.integers(0, v.shape[1], 6)] = np.array([0x7f80, 0xff80] * 3, np.uint16)
+    x = synth.activations(975, T, H)
+    kind = r.integers(0, 4, x.shape)                   # 0: one bf16, 1: two of them, 2: zero, 3: as drawn
+    x[kind == 0] = (x[kind == 0].view(np.uint32) & 0xffff0000).view(np.float32)
+    x[kind == 1] = (x[kind == 1].view(np.uint32) & 0xffffff00).view(np.float32)
+    x[(kind == 2) & (r.random(x.shape) < 0.1)] = 0.0
+    lg = synth.uniform_logits(976, T, E)
+    with mlamoe.Context(0) as ctx:
+        ctx.moe_init(H, E, NS, K, I)
+        ctx.moe_load_layer(0, w, mlamoe.MM_LOAD_BF16)
+        out = ctx.moe_forward(0, x, logits=lg)[0]
+        ref = np.concatenate([ctx.moe_forward(0, x[t:t + 4], logits=lg[t:t + 4])[0] for t in range(0, T, 4)])
+    assert np.isinf(ref).any() or where in ("eg", "sg")     # (silu(-inf) is NaN: so are the rows it meets)
+    fin = np.isfinite(ref)
+    assert np.array_equal(np.isfinite(out), fin) and np.array_equal(out[~fin], ref[~fin], equal_nan=True)
+    assert np.linalg.norm(out[fin] - ref[fin]) <= 2 * TOL * np.linalg.norm(ref[fin])
+
+
+@pytest.mark.parametrize("e", [-100, -110, -117])
+def test_small_activations(e):
+    """A value whose lower bf16 parts are subnormal: still the whole of it."""
+    H, E, K, I, NS, T = 64, 2, 1, 64, 0, 20
+    w = synth.moe_layer(977, H, E, I, NS)
+    for k in ("eg", "eu", "ed"):
+        w[k] = np.zeros_like(w[k])
+    one = np.uint16(0x3f80)
+    w["eu"][:, 0, 0] = w["eg"][:, 0, 1] = one          # u[0] = x[0], g[0] = x[1]
+    w["ed"][:, :, 0] = np.uint16(0x7100)               # out = 2^99 h[0]: h's own parts are normal
+    x = np.zeros((T, H), np.float32)
+    x[:, 0] = np.ldexp(1.0 + np.random.default_rng(978).integers(1, 1 << 23, T) / (1 << 23), e).astype(np.float32)
+    x[:, 1] = 2.0 ** 30                                # silu(2^30) = 2^30
+    with mlamoe.Context(0) as ctx:
+        ctx.moe_init(H, E, NS, K, I)
+        ctx.moe_load_layer(0, w, mlamoe.MM_LOAD_BF16)
+        out, idx, wt, _ = ctx.moe_forward(0, x, logits=synth.uniform_logits(979, T, E))
+    want = wt[:, 0].astype(np.float64) * x[:, 0] * 2.0 ** 129
+    print(f"2^{e}: {np.max(np.abs(out / want[:, None] - 1)):.2e}", flush=True)
+    assert np.max(np.abs(out / want[:, None] - 1)) < max(2.0 ** -22, 2.0 ** (-132 - e))
+
+
 def test_rows_past_32_bit_offsets():
     """An intermediate size at which 64 hidden rows span 4 GB: the call takes
     the GEMV stages.  The experts' weights are zero but for a few rows."""
