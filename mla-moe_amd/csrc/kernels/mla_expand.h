@@ -50,11 +50,15 @@ __device__ __forceinline__ f32x16 mfma32(i32x4 a, i32x4 b, f32x16 c) {
 /* Keys (part 0) or values (part 1) of 128 cache rows and one head: 128 x 128
  * x 512, four multiplying waves (2 x 2, 64 x 64 each) and four loading, a
  * ring of XNS chunks of 64 latent values; two blocks per CU, one's products
- * and output beside the other's loads (2,048 keys, 16 heads: 22 us; one block
- * per CU with four chunks in flight 31).  The pairs leave through LDS in
- * whole lines: as 8-byte stores from the accumulators 32.  Rows at or past the tile's length
- * are zeros: a value of an unwritten cache row must not meet a probability
- * of zero as an infinity. */
+ * and output beside the other's loads.  16 heads: one prompt of 2,048 rows
+ * (512 blocks, two per CU) 20 us; prompts of 1,364 and 683 rows (544 blocks:
+ * 32 run in a second turn) 24.  Which operand comes first is a matter of
+ * addresses: as a choice at each product it took a branch each and spilled 10
+ * registers (23 and 33 us).  In that form one block per CU with four chunks in
+ * flight took 31 us for the 2,048 rows, and the pairs stored from the
+ * accumulators, 8 bytes at a time, 32: they leave through LDS in whole lines.
+ * Rows at or past the tile's length are zeros: a value of an unwritten cache
+ * row must not meet a probability of zero as an infinity. */
 #define XNS MM_MLA_XNS
 extern "C" __global__ __launch_bounds__(512, 4) void mm_mla_expand(mm_mla_expand_args a) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t xlds[];
@@ -95,7 +99,12 @@ extern "C" __global__ __launch_bounds__(512, 4) void mm_mla_expand(mm_mla_expand
         VMCNT_WAIT(0);
     } else {
         const int wm = wave >> 1, wn = wave & 1, c32 = lane & 31, hi = lane >> 5;
-        f32x16 acc[2][2] = {};                             /* [key tile][column tile] */
+        /* the first operand's rows are a result's registers, the second's its
+         * lanes: keys have lanes for keys (the weights first), values lanes for
+         * dims (the latent rows first) -- one code for both, by the addresses */
+        const uint32_t ax = (uint32_t)(64 * wm * 128), aw = (uint32_t)(16384 + 64 * wn * 128);
+        const uint32_t a0 = part == 0 ? aw : ax, a1 = part == 0 ? ax : aw;
+        f32x16 acc[2][2] = {};                             /* [first operand's tile][second's] */
 #pragma unroll
         for (int c = 0; c < NC; c++) {
             __builtin_amdgcn_s_barrier();
@@ -104,17 +113,16 @@ extern "C" __global__ __launch_bounds__(512, 4) void mm_mla_expand(mm_mla_expand
 #pragma unroll
             for (int s = 0; s < 4; s++) {
                 const uint32_t p = 16 * ((2 * s + hi) ^ ((c32 >> 1) & 7));
-                i32x4 x[2], w[2];
+                i32x4 f0[2], f1[2];
 #pragma unroll
                 for (int t = 0; t < 2; t++) {
-                    x[t] = *(lds_c4)(sb + p + (64 * wm + 32 * t) * 128);
-                    w[t] = *(lds_c4)(sb + p + 16384 + (64 * wn + 32 * t) * 128);
+                    f0[t] = *(lds_c4)(sb + p + a0 + 32 * t * 128);
+                    f1[t] = *(lds_c4)(sb + p + a1 + 32 * t * 128);
                 }
 #pragma unroll
-                for (int t = 0; t < 2; t++)
+                for (int u = 0; u < 2; u++)
 #pragma unroll
-                    for (int j = 0; j < 2; j++)            /* keys: lanes are keys; values: lanes are dims */
-                        acc[t][j] = part == 0 ? mfma32(w[j], x[t], acc[t][j]) : mfma32(x[t], w[j], acc[t][j]);
+                    for (int v = 0; v < 2; v++) acc[u][v] = mfma32(f0[u], f1[v], acc[u][v]);
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         }
@@ -122,22 +130,21 @@ extern "C" __global__ __launch_bounds__(512, 4) void mm_mla_expand(mm_mla_expand
          * load landed, every read done), then out in whole lines */
         __builtin_amdgcn_s_barrier();
 #pragma unroll
-        for (int t = 0; t < 2; t++)
+        for (int u = 0; u < 2; u++)
 #pragma unroll
-            for (int j = 0; j < 2; j++)
+            for (int v = 0; v < 2; v++)
 #pragma unroll
                 for (int g = 0; g < 4; g++) {
                     typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
                     uint32_t h0, h1, l0, l1;
-                    split_pk(acc[t][j][4 * g], acc[t][j][4 * g + 1], &h0, &l0);
-                    split_pk(acc[t][j][4 * g + 2], acc[t][j][4 * g + 3], &h1, &l1);
-                    uint32_t o = (uint32_t)((2 * wm + t) * 2 * XT);
-                    if (part == 0) {                   /* key c32, dims 64 wn + 32 j + 8 g + 4 hi .. + 3 */
-                        o += c32 * 256 + 16 * (((64 * wn + 32 * j) / 8 + g) ^ (c32 & 15)) + 8 * hi;
-                    } else {                           /* dim, keys 8 g + 4 hi .. + 3 */
-                        const int d = 64 * wn + 32 * j + c32;
-                        o += d * 64 + 16 * ((2 * (g >> 1) + hi) ^ ((d >> 2) & 3)) + 8 * (g & 1);
-                    }
+                    split_pk(acc[u][v][4 * g], acc[u][v][4 * g + 1], &h0, &l0);
+                    split_pk(acc[u][v][4 * g + 2], acc[u][v][4 * g + 3], &h1, &l1);
+                    /* key c32 of tile v, dims 64 wn + 32 u + 8 g + 4 hi .. + 3 */
+                    const uint32_t ok = (2 * wm + v) * 2 * XT + c32 * 256 + 16 * (((64 * wn + 32 * u) / 8 + g) ^ (c32 & 15)) + 8 * hi;
+                    /* dim d, keys 8 g + 4 hi .. + 3 of tile u */
+                    const int d = 64 * wn + 32 * v + c32;
+                    const uint32_t ov = (2 * wm + u) * 2 * XT + d * 64 + 16 * ((2 * (g >> 1) + hi) ^ ((d >> 2) & 3)) + 8 * (g & 1);
+                    const uint32_t o = part == 0 ? ok : ov;
                     *(u32x2 *)(xlds + o) = (u32x2){h0, h1};
                     *(u32x2 *)(xlds + o + XT) = (u32x2){l0, l1};
                 }
