@@ -238,12 +238,14 @@ int mm_mla_expanded_rows(mm_ctx *c, int layer, const float *q, const uint16_t *c
                          const int32_t *ktiles, int nkt, const int32_t *qtiles, int nqt, int nblk,
                          float *ctx_out) {
     const int NH = c->mla.n_heads;
+    const size_t n = (size_t)nblk * NH;
     uint8_t *kv;
-    int st = mm_workspace(c, (size_t)nblk * NH * MM_MLA_XBLK, (void **)&kv);
+    int st = mm_workspace(c, n * (MM_MLA_XBLK + 4), (void **)&kv);
     if (st) return st;
-    mm_mla_expand_args ea = {cache, c->mla_kvb[layer], kv, ktiles, seq_stride, NH};
+    uint32_t *nf = (uint32_t *)(kv + n * MM_MLA_XBLK);
+    mm_mla_expand_args ea = {cache, c->mla_kvb[layer], kv, nf, ktiles, seq_stride, NH};
     if ((st = mm_launch(c, K_MLA_EXPAND, (unsigned)NH, 2, (unsigned)nkt, 512, MM_MLA_XEXP_LDS, &ea))) return st;
-    mm_mla_xattn_args xa = {q, cache, kv, qtiles, ctx_out, seq_stride, NH, c->mla.softmax_scale};
+    mm_mla_xattn_args xa = {q, cache, kv, nf, qtiles, ctx_out, seq_stride, NH, c->mla.softmax_scale};
     return mm_launch(c, K_MLA_ATTN_X, (unsigned)nqt * (unsigned)NH, 1, 1, 256, MM_MLA_XATTN_LDS, &xa);
 }
 

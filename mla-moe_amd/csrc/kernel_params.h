@@ -473,6 +473,7 @@ typedef struct {
     const uint16_t *cache;    /* [sequences, seq_stride, KVL + QKR] */
     const uint16_t *kv_b;     /* [NH, W_UK 128 rows | W_UV 128 rows, KVL] */
     uint8_t *kv;              /* [blocks][NH] blocks of MM_MLA_XBLK bytes */
+    uint32_t *nf;             /* [blocks][NH] bit per key: some value of its was not finite */
     const int32_t *tiles;     /* per 128 keys: slot, first key, sequence length, first block */
     int seq_stride, NH;
 } mm_mla_expand_args;
@@ -480,6 +481,7 @@ typedef struct {
     const float *q;           /* [R, NH, 128 + QKR] */
     const uint16_t *cache;
     const uint8_t *kv;
+    const uint32_t *nf;
     const int32_t *tiles;     /* per 64 rows: first row, rows, first position, slot, first block */
     float *ctx;               /* [R, NH * 128] */
     int seq_stride, NH;

@@ -42,6 +42,11 @@ __device__ __forceinline__ void split_pk(float a, float b, uint32_t *hi, uint32_
     *lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a - bf16_lo(w), b - bf16_hi(w)}, bf16x2));
 }
 
+/* Bits 15 and 31: whether the low and the high bf16 of a word are not finite. */
+__device__ __forceinline__ uint32_t nonfinite2(uint32_t w) {
+    return ((w & 0x7f807f80u) + 0x00800080u) & 0x80008000u;
+}
+
 __device__ __forceinline__ f32x16 mfma32(i32x4 a, i32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
                                                    0, 0, 0);
@@ -156,8 +161,39 @@ extern "C" __global__ __launch_bounds__(512, 4) void mm_mla_expand(mm_mla_expand
     if (kb * XB >= len) return;
     uint8_t *dst = a.kv + ((size_t)(blk0 + kb) * a.NH + h) * XBLK + part * 2 * XT + (wave & 1) * XT;
     const uint8_t *src = xlds + b * 2 * XT + (wave & 1) * XT;
+    u32x4 v[XT / 1024];
+    uint32_t any = 0;
 #pragma unroll
-    for (int u = 0; u < XT / 1024; u++) *(u32x4 *)(dst + u * 1024 + lane * 16) = *(const u32x4 *)(src + u * 1024 + lane * 16);
+    for (int u = 0; u < XT / 1024; u++) {
+        v[u] = *(const u32x4 *)(src + u * 1024 + lane * 16);
+        any |= nonfinite2(v[u].x) | nonfinite2(v[u].y) | nonfinite2(v[u].z) | nonfinite2(v[u].w);
+    }
+    if (part == 1) {
+        /* zero times a later key's infinity or NaN must not reach the rows
+         * before it: such a value is stored as zero (its low part is no number
+         * either) and its key's bit set, for the rows that do see it */
+        uint32_t keys = 0;
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(any != 0) != 0, 0)) {
+#pragma unroll 1
+            for (int u = 0; u < XT / 1024; u++) {
+                const int d = 16 * u + (lane >> 2), p = (lane & 3) ^ ((d >> 2) & 3);
+                u32x4 w = *(const u32x4 *)(src + u * 1024 + lane * 16);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const uint32_t n = nonfinite2(w[i]);
+                    w[i] &= ~((n >> 15) * 0xffffu);
+                    keys |= ((n >> 15 & 1u) | (n >> 30 & 2u)) << (16 * (p >> 1) + 4 * (p & 1) + 2 * (i & 1) + 8 * (i >> 1));
+                }
+                *(u32x4 *)(dst + u * 1024 + lane * 16) = w;
+            }
+#pragma unroll
+            for (int off = 1; off < MM_WAVE; off <<= 1) keys |= (uint32_t)__shfl_xor((int)keys, off, MM_WAVE);
+        }
+        if (lane == 0 && (wave & 1) == 0) a.nf[(size_t)(blk0 + kb) * a.NH + h] = keys;
+        if (keys) return;
+    }
+#pragma unroll
+    for (int u = 0; u < XT / 1024; u++) *(u32x4 *)(dst + u * 1024 + lane * 16) = v[u];
 }
 
 /* Flash attention of 64 rows (consecutive positions of one sequence) and one
@@ -232,6 +268,17 @@ extern "C" __global__ __launch_bounds__(256, 2) void mm_mla_attn_expanded(mm_mla
     }
     const int pos = pos0 + min(myrow, nrows - 1);      /* this lane's row */
     const int wlast = pos0 + min(32 * wr + 31, nrows - 1), wfirst = pos0 + min(32 * wr, nrows - 1);
+    /* the first key with a value that is not finite (mm_mla_expand stored
+     * zeros): the rows that see it give NaN, as its infinity or NaN would */
+    int kbad = INT32_MAX;
+    for (int b0 = 0; b0 < nblk && kbad == INT32_MAX; b0 += MM_WAVE) {
+        const uint32_t nf = b0 + lane < nblk ? a.nf[(size_t)(blk0 + b0 + lane) * a.NH + h] : 0;
+        const uint64_t any = __builtin_amdgcn_ballot_w64(nf != 0);
+        if (any) {
+            const int f = __builtin_ctzll(any);
+            kbad = XB * (b0 + f) + __builtin_ctz(__builtin_amdgcn_readlane((int)nf, f));
+        }
+    }
     const float scale2 = a.scale * 1.44269504088896341f;   /* scores in units of ln 2: e^x is one v_exp */
     float m = -INFINITY, l = 0.0f;
     f32x16 O[4] = {};
@@ -330,6 +377,7 @@ extern "C" __global__ __launch_bounds__(256, 2) void mm_mla_attn_expanded(mm_mla
         asm volatile("" ::: "memory");
     }
     asm volatile("" ::: "memory");
+    if (pos >= kbad) l = __builtin_nanf("");
 
     /* the odd blocks' (m, l, O) to the wave of the same rows; both halves of a
      * row's lanes hold the same m, each its own share of l */

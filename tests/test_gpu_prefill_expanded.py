@@ -82,3 +82,33 @@ def test_scratch_cap_falls_back(model, monkeypatch):
     a = logits(model, steps, monkeypatch, 128)
     b = logits(model, steps, monkeypatch, 0)
     assert np.linalg.norm(a - b) < 2e-4 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("first,n,bad", [(0, 150, 149), (0, 150, 100), (0, 150, 63), (37, 129, 40), (37, 129, 128),
+                                         (0, 700, 350)])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_row_that_is_not_finite(model, first, n, bad, value):
+    """A row whose embedding is not finite gives NaN from its position on, and
+    leaves the rows before it as they are: a key that a row does not see
+    weighs nothing, whatever it holds."""
+    m = dict(model, embed=model["embed"].copy())
+    m["embed"][299] = synth.bf16_from_f32(np.full(CFG["H"], value, np.float32))
+    toks = np.random.default_rng(6).integers(0, 299, first + n).astype(np.int32)
+    out = []
+    with mlamoe.Context(0) as ctx:
+        eng = Engine.from_host(ctx, CFG, m, mlamoe.rope_inv_freq(64, 10000.0), max_batch=1, max_seq=1200, max_rows=2048)
+        try:
+            if first:
+                eng.step_rows(np.zeros(first), toks[:first], np.arange(first), [])
+            for t in (toks[first + bad], 299):
+                toks[first + bad] = t
+                ctx.prof_reset()
+                ctx.prof_enable(True)
+                out.append(eng.step_rows(np.zeros(n), toks[first:], np.arange(first, first + n), np.arange(n),
+                                         want_logits=True)[1])
+                assert ctx.prof_query("mm_mla_attn_expanded")[1] == CFG["n_layers"]
+        finally:
+            ctx.prof_enable(False)
+            eng.close()
+    assert np.array_equal(out[0][:bad], out[1][:bad])
+    assert np.isfinite(out[0]).all() and np.isnan(out[1][bad:]).all()
