@@ -201,6 +201,10 @@ int mm_ctx_create(int device, mm_ctx **out) {
     c->moe_t_chunk = 0;
     ev = getenv("MLAMOE_MOE_T_CHUNK");
     if (ev && *ev && atoi(ev) > 0) c->moe_t_chunk = atoi(ev);
+    /* MLAMOE_WS_MAX (bytes): the workspace grows no further, as if the GPU
+     * were full */
+    ev = getenv("MLAMOE_WS_MAX");
+    if (ev && *ev && atoll(ev) > 0) c->ws_max = (size_t)atoll(ev);
     if ((st = mm_noalloc_setup(c))) goto fail;
     *out = c;
     return MM_OK;
@@ -388,8 +392,23 @@ int mm_workspace(mm_ctx *c, size_t bytes, void **out) {
         if (c->ws) MM_HIP(hipFree(c->ws));
         c->ws = NULL;
         c->ws_bytes = 0;
+        /* a quarter to spare; without it where that cannot be had */
         size_t nb = bytes + bytes / 4;
-        MM_HIP(hipMalloc(&c->ws, nb));
+        if (c->ws_max && nb > c->ws_max) nb = c->ws_max > bytes ? c->ws_max : bytes;
+        hipError_t e = hipErrorOutOfMemory;
+        if (!c->ws_max || bytes <= c->ws_max) {
+            e = hipMalloc(&c->ws, nb);
+            if (e == hipErrorOutOfMemory && nb > bytes) {
+                (void)hipGetLastError();
+                e = hipMalloc(&c->ws, nb = bytes);
+            }
+        }
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            c->ws = NULL;
+            return mm_fail(e == hipErrorOutOfMemory ? MM_ERR_NOMEM : MM_ERR_HIP, "workspace of %zu bytes: %s", bytes,
+                           hipGetErrorString(e));
+        }
         c->ws_bytes = nb;
     }
     *out = c->ws;

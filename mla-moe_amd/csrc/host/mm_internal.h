@@ -153,6 +153,7 @@ struct mm_ctx {
     /* growable device workspace */
     void *ws;
     size_t ws_bytes;
+    size_t ws_max;              /* bytes the workspace may have (0: what the GPU has) */
     /* growable device staging of the synchronous host-pointer entry points */
     void *io;
     size_t io_bytes;

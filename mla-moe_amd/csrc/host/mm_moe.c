@@ -628,23 +628,29 @@ static int bf16_mm_pass(mm_ctx *c, const mm_moe_layer *L, int T, const float *xn
     return MM_OK;
 }
 
-/* bf16 weights as grouped GEMMs (kernels/moe_bf16_mm.h), in passes of at
- * most MM_BF16_MM_T_CHUNK tokens, or of as many as a fixed workspace holds
- * (a token's results do not depend on the pass it is in).  *fits is 0, and
- * nothing has run, when the fixed workspace cannot hold one token. */
+/* bf16 weights as grouped GEMMs (kernels/moe_bf16_mm.h), in even passes of at
+ * most MM_BF16_MM_T_CHUNK tokens and MM_BF16_MM_WS bytes, or of as many tokens
+ * as a fixed workspace or the GPU's free memory holds (a token's results do
+ * not depend on the pass it is in).  *fits is 0, and nothing has run, when that
+ * is fewer than MM_BF16_MM_MIN_T. */
 static int forward_bf16_mm(mm_ctx *c, const mm_moe_layer *L, int T, const float *xn, float *out,
                            const float *logits, int32_t *idx, float *wts, float *probs, int acc,
                            const mm_fixed_ws *fx, int *fits) {
     const mm_moe_config *g = &c->moe;
     const size_t H = g->hidden_size, E = g->n_routed_experts, K = g->n_experts_per_tok;
-    int tc = T < MM_BF16_MM_T_CHUNK ? T : MM_BF16_MM_T_CHUNK;
-    if (fx)
-        while (tc > 0 && bf16_mm_layout(g, tc, logits != NULL).bytes > fx->cap) tc -= (tc + 15) / 16;
-    *fits = tc > 0;
+    const size_t cap = fx ? fx->cap : MM_BF16_MM_WS;
+    int tc = T < MM_BF16_MM_T_CHUNK ? T : MM_BF16_MM_T_CHUNK, st = MM_OK;
+    while (tc >= MM_BF16_MM_MIN_T && bf16_mm_layout(g, tc, logits != NULL).bytes > cap) tc -= (tc + 15) / 16;
+    bf16_mm_plan w;
+    char *ws = NULL;
+    for (; tc >= MM_BF16_MM_MIN_T; tc /= 2) {
+        const int passes = (T + tc - 1) / tc;
+        tc = (T + passes - 1) / passes;
+        w = bf16_mm_layout(g, tc, logits != NULL);
+        if ((st = take_ws(c, fx, w.bytes, &ws)) != MM_ERR_NOMEM) break;
+    }
+    *fits = tc >= MM_BF16_MM_MIN_T;
     if (!*fits) return MM_OK;
-    const bf16_mm_plan w = bf16_mm_layout(g, tc, logits != NULL);
-    char *ws;
-    int st = take_ws(c, fx, w.bytes, &ws);
     for (int t0 = 0; t0 < T && !st; t0 += tc)
         st = bf16_mm_pass(c, L, T - t0 < tc ? T - t0 : tc, xn + (size_t)t0 * H, out + (size_t)t0 * H,
                           logits ? logits + (size_t)t0 * E : NULL, idx ? idx + (size_t)t0 * K : NULL,

@@ -87,7 +87,10 @@ typedef struct {
 #ifndef MM_BF16_MM_MIN_T
 #define MM_BF16_MM_MIN_T 5
 #endif
-#define MM_BF16_MM_T_CHUNK 2048   /* rows of one pass (its workspace: ~180 KB per row) */
+/* Rows of one pass, and bytes of its workspace: 180 KB per row at DeepSeek-V2-Lite's
+ * sizes (370 MB), 750 KB at a hidden size of 7,168 with 8 experts of 2,048 per token. */
+#define MM_BF16_MM_T_CHUNK 2048
+#define MM_BF16_MM_WS ((size_t)1 << 30)
 #define MM_BF16_MM_GRID 256       /* persistent grid: one block per CU */
 #define MM_BF16_MM_THREADS 512    /* four multiplying waves, two loading weights, two activations */
 /* The load rings of 16-, 32- and 64-row tiles (dynamic LDS): NSW stages of KB

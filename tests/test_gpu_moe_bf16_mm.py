@@ -97,6 +97,36 @@ def test_fixed_workspace():
         assert np.array_equal(a.download(), b.download())
 
 
+@pytest.mark.parametrize("ws_max,gemv", [(16 << 20, False), (3 << 20, False), (1 << 19, True)])
+def test_workspace_that_cannot_grow(monkeypatch, ws_max, gemv):
+    """When the GPU has no room for a pass's workspace the call runs in
+    shorter passes (the same bits), and without room for 5 tokens by the
+    GEMV stages."""
+    H, E, K, I, NS, T = 1024, 8, 4, 512, 2, 300
+    w, x = synth.moe_layer(985, H, E, I, NS), synth.activations(986, T, H)
+    outs = []
+    for limit in (None, ws_max):
+        if limit:
+            monkeypatch.setenv("MLAMOE_WS_MAX", str(limit))
+        else:
+            monkeypatch.delenv("MLAMOE_WS_MAX", raising=False)
+        with mlamoe.Context(0) as ctx:
+            ctx.moe_init(H, E, NS, K, I)
+            ctx.moe_load_layer(0, w, mlamoe.MM_LOAD_BF16)
+            ctx.prof_enable(True)
+            out, idx, wt, _ = ctx.moe_forward(0, x)
+            outs.append(out)
+            grouped = ctx.prof_query("mm_bf16_rows")[1]
+            ctx.prof_enable(False)
+            assert ctx.workspace_bytes() <= ws_max if limit else ctx.workspace_bytes() > 16 << 20
+            assert grouped == 1 if not limit else grouped == 0 if gemv else grouped > 1
+    if gemv:
+        ref = ref64(w, x, idx, wt, NS)
+        assert np.linalg.norm(outs[1] - ref) < TOL * np.linalg.norm(ref)
+    else:
+        assert np.array_equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("inf", [False, True])
 def test_large_and_infinite_activations(inf):
     """Activations near the largest fp32 value split without overflow; an
