@@ -425,7 +425,8 @@ static int run_planned(mm_engine *e, int R, int n_want, int32_t *next, float *lo
     int32_t *hio = e->h_io;
     int st;
     const int NH = c->mla.n_heads, QD = NH * (c->mla.qk_nope_head_dim + c->mla.qk_rope_head_dim);
-    if (p->nqt)
+    int expand = p->nqt > 0;
+    if (expand)
         MM_HIP(hipMemcpyAsync(e->xt_d, e->xt_h, XT_BYTES, hipMemcpyHostToDevice, c->stream));
     int32_t *d_tok = e->d_io + IO_TOK * MR, *d_pos = e->d_io + IO_POS * MR;
     int32_t *d_len = e->d_io + IO_LEN * MR, *d_slot = e->d_io + IO_SLOT * MR;
@@ -448,11 +449,17 @@ static int run_planned(mm_engine *e, int R, int n_want, int32_t *next, float *lo
                                     fuse ? e->fcomp : NULL,
                                     fuse ? &ra : NULL)))
             return st;
-        if (p->nqt && (st = mm_mla_expanded_rows(c, l, e->q, e->cache[l], e->lcap[l], e->xt_d, p->nkt,
-                                                 e->xt_d + 4 * XT_MAX, p->nqt, p->nblk, e->ctxo)))
-            return st;
-        for (int i = 0; i < p->n_abs; i++) {
-            const int r0 = p->abs[2 * i], n = p->abs[2 * i + 1] - r0;
+        /* expanded rows first, then the others' ranges; all of them as one
+         * absorbed range when the GPU has no room for the expanded keys */
+        if (expand) {
+            st = mm_mla_expanded_rows(c, l, e->q, e->cache[l], e->lcap[l], e->xt_d, p->nkt, e->xt_d + 4 * XT_MAX,
+                                      p->nqt, p->nblk, e->ctxo);
+            if (st && st != MM_ERR_NOMEM) return st;
+            expand = !st;
+        }
+        const int whole[2] = {0, R}, *range = p->nqt && !expand ? whole : p->abs;
+        for (int i = 0; i < (range == whole ? 1 : p->n_abs); i++) {
+            const int r0 = range[2 * i], n = range[2 * i + 1] - r0;
             int kvlen = 1;     /* the range's longest context */
             for (int r = r0; r < r0 + n; r++)
                 if (hio[IO_LEN * MR + r] > kvlen) kvlen = hio[IO_LEN * MR + r];

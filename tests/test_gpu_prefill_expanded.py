@@ -84,6 +84,37 @@ def test_scratch_cap_falls_back(model, monkeypatch):
     assert np.linalg.norm(a - b) < 2e-4 * np.linalg.norm(b)
 
 
+def test_no_room_for_the_expanded_keys(monkeypatch):
+    """A step whose expanded keys the GPU has no room for takes the absorbed
+    form.  64 heads: 512 rows take 134 MB of absorbed scratch, their expanded
+    keys 33.5 MB per 512 positions."""
+    c = dict(CFG, NH=64)
+    m = synth.model(4322, c["n_layers"], c["first_dense"], c["H"], c["NH"], c["QKN"], c["QKR"], c["KVL"], c["VHD"],
+                    c["dense_inter"], c["E"], c["I"], c["n_shared"], c["vocab"])
+    toks = np.random.default_rng(7).integers(0, c["vocab"], 3072).astype(np.int32)
+    out, forms = [], []
+    for limit in (None, 150 << 20):
+        if limit:
+            monkeypatch.setenv("MLAMOE_WS_MAX", str(limit))
+        with mlamoe.Context(0) as ctx:
+            eng = Engine.from_host(ctx, c, m, mlamoe.rope_inv_freq(64, 10000.0), max_batch=1, max_seq=3072,
+                                   init_seq=3072, max_rows=512)
+            try:
+                ctx.prof_enable(True)
+                for p0 in range(0, 3072, 512):
+                    ctx.prof_reset()
+                    lg = eng.step_rows(np.zeros(512), toks[p0:p0 + 512], np.arange(p0, p0 + 512), np.arange(512),
+                                       want_logits=True)[1]
+                    forms.append(ctx.prof_query("mm_mla_attn_expanded")[1])
+                assert not limit or ctx.workspace_bytes() <= limit
+                ctx.prof_enable(False)
+            finally:
+                eng.close()
+        out.append(lg.astype(np.float64))
+    assert forms == [2] * 6 + [2] * 4 + [0] * 2
+    assert np.linalg.norm(out[0] - out[1]) < 2e-4 * np.linalg.norm(out[0])
+
+
 @pytest.mark.parametrize("first,n,bad", [(0, 150, 149), (0, 150, 100), (0, 150, 63), (37, 129, 40), (37, 129, 128),
                                          (0, 700, 350)])
 @pytest.mark.parametrize("value", [np.nan, np.inf])
