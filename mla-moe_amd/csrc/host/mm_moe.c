@@ -11,7 +11,6 @@
 
 #include "mm_internal.h"
 
-#define BF16_NT_MAX 8         /* tokens per pass of the bf16 GEMV path */
 #define GU_ROWS_PER_BLOCK 4   /* stage 1: one gate/up row pair per wave */
 #define GU2_ROWS_PER_BLOCK 8  /* stage 2: two row pairs per wave (one round of loads) */
 #define RSH_ROWS_PER_BLOCK 16 /* shared gate/up beside the router: four row pairs per wave */
@@ -545,6 +544,19 @@ static int bf16_mm_ok(const mm_moe_config *g) {
     return w * H < 0x7FFF0000u && 64 * (w > H ? w : H) < 0x7FFF0000u;
 }
 
+/* Whether passes of T tokens are faster as grouped GEMMs (kernel_params.h has
+ * the measurements).  The routing is not known here: K different experts per
+ * token, each as likely as any other, touch E (1 - (1 - K / E)^T). */
+static int bf16_mm_pays(const mm_moe_config *g, int T) {
+    const double E = g->n_routed_experts, K = g->n_experts_per_tok, NS = g->n_shared_experts;
+    if (T > MM_BF16_NT_MAX) return 1;
+    if (T < MM_BF16_MM_MIN_T || E > 64) return 0;
+    double untouched = E;
+    for (int t = 0; t < T; t++) untouched *= 1 - K / E;
+    const double saved = T * K - (E - untouched) + (T - 1) * NS;      /* experts not read again */
+    return saved * 6 * g->hidden_size * g->moe_inter_size >= MM_BF16_MM_SAVED;
+}
+
 /* One pass over T tokens: router logits, routing with per-expert row lists,
  * the sorted planes of x, gate/up, down, combine. */
 static int bf16_mm_pass(mm_ctx *c, const mm_moe_layer *L, int T, const float *xn, float *out,
@@ -631,8 +643,8 @@ static int bf16_mm_pass(mm_ctx *c, const mm_moe_layer *L, int T, const float *xn
 /* bf16 weights as grouped GEMMs (kernels/moe_bf16_mm.h), in even passes of at
  * most MM_BF16_MM_T_CHUNK tokens and MM_BF16_MM_WS bytes, or of as many tokens
  * as a fixed workspace or the GPU's free memory holds (a token's results do
- * not depend on the pass it is in).  *fits is 0, and nothing has run, when that
- * is fewer than MM_BF16_MM_MIN_T. */
+ * not depend on the pass it is in).  *fits is 0, and nothing has run, when so
+ * short passes do not pay. */
 static int forward_bf16_mm(mm_ctx *c, const mm_moe_layer *L, int T, const float *xn, float *out,
                            const float *logits, int32_t *idx, float *wts, float *probs, int acc,
                            const mm_fixed_ws *fx, int *fits) {
@@ -643,13 +655,13 @@ static int forward_bf16_mm(mm_ctx *c, const mm_moe_layer *L, int T, const float 
     while (tc >= MM_BF16_MM_MIN_T && bf16_mm_layout(g, tc, logits != NULL).bytes > cap) tc -= (tc + 15) / 16;
     bf16_mm_plan w;
     char *ws = NULL;
-    for (; tc >= MM_BF16_MM_MIN_T; tc /= 2) {
+    for (; bf16_mm_pays(g, tc); tc /= 2) {
         const int passes = (T + tc - 1) / tc;
         tc = (T + passes - 1) / passes;
         w = bf16_mm_layout(g, tc, logits != NULL);
         if ((st = take_ws(c, fx, w.bytes, &ws)) != MM_ERR_NOMEM) break;
     }
-    *fits = tc >= MM_BF16_MM_MIN_T;
+    *fits = bf16_mm_pays(g, tc);
     if (!*fits) return MM_OK;
     for (int t0 = 0; t0 < T && !st; t0 += tc)
         st = bf16_mm_pass(c, L, T - t0 < tc ? T - t0 : tc, xn + (size_t)t0 * H, out + (size_t)t0 * H,
@@ -659,8 +671,8 @@ static int forward_bf16_mm(mm_ctx *c, const mm_moe_layer *L, int T, const float 
     return st;
 }
 
-/* bf16 weights: grouped GEMMs from MM_BF16_MM_MIN_T tokens on, else the GEMV
- * stages (kernels/moe_bf16.hip), BF16_NT_MAX tokens per pass. */
+/* bf16 weights: grouped GEMMs where they pay, else the GEMV
+ * stages (kernels/moe_bf16.hip), MM_BF16_NT_MAX tokens per pass. */
 static int forward_bf16(mm_ctx *c, const mm_moe_layer *L, int T, const float *xn, float *out,
                         const float *logits, int32_t *idx, float *wts, float *probs, int acc,
                         const mm_fixed_ws *fx) {
@@ -669,13 +681,13 @@ static int forward_bf16(mm_ctx *c, const mm_moe_layer *L, int T, const float *xn
     const int I = g->moe_inter_size, S = g->n_shared_experts * I;
     const size_t hw = (size_t)K * I + S;
     const int wide = E > MM_EMAX_FAST;
-    if (T >= MM_BF16_MM_MIN_T && bf16_mm_ok(g)) {
+    if (bf16_mm_pays(g, T) && bf16_mm_ok(g)) {
         int fits;
         const int st = forward_bf16_mm(c, L, T, xn, out, logits, idx, wts, probs, acc, fx, &fits);
         if (st || fits) return st;
     }
     mm_plan p = {0};
-    const size_t o_h = plan_take(&p, (size_t)BF16_NT_MAX * hw * sizeof(float));
+    const size_t o_h = plan_take(&p, (size_t)MM_BF16_NT_MAX * hw * sizeof(float));
     const size_t o_i = plan_take(&p, (size_t)T * K * sizeof(int32_t));
     const size_t o_w = plan_take(&p, (size_t)T * K * sizeof(float));
     /* router logits scratch: the wide routers', or the split router's of
@@ -694,8 +706,8 @@ static int forward_bf16(mm_ctx *c, const mm_moe_layer *L, int T, const float *xn
         if ((st = route_wide(c, L, T, xn, logits, (float *)(ws + o_lg), idx, wts, probs, NULL)))
             return st;
     }
-    for (int t0 = 0; t0 < T; t0 += BF16_NT_MAX) {
-        const int Tc = T - t0 < BF16_NT_MAX ? T - t0 : BF16_NT_MAX;
+    for (int t0 = 0; t0 < T; t0 += MM_BF16_NT_MAX) {
+        const int Tc = T - t0 < MM_BF16_NT_MAX ? T - t0 : MM_BF16_NT_MAX;
         mm_gu_bf16_args a;
         memset(&a, 0, sizeof(a));
         a.r.x = xn + (size_t)t0 * H;

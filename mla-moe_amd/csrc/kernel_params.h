@@ -80,13 +80,26 @@ typedef struct {
     int rows_per_block;
 } mm_down_bf16_args;
 
-/* bf16 MoE as grouped GEMMs (moe_bf16_mm.h), from MM_BF16_MM_MIN_T tokens
- * on: the GEMV streams an expert once per token that chose it, the GEMMs once
- * per row tile but through six launches (DeepSeek-V2-Lite layer, 4 tokens: 98
- * us by GEMV, 103 by GEMM; 5: 127 and 115; 8: 186 and 143; 64: 1430 and 248). */
+/* bf16 MoE as grouped GEMMs (moe_bf16_mm.h) above MM_BF16_NT_MAX tokens, where
+ * the GEMV stages would take a second pass, and from MM_BF16_MM_MIN_T tokens
+ * on where sharing is expected to save MM_BF16_MM_SAVED bytes of weights: the
+ * GEMV streams an expert once per token that chose it, the GEMMs once per row
+ * tile, but through six launches and at 4-5 TB/s instead of 6.  Up to 64
+ * experts only: with more, few tokens share one, and the GEMV stages have the
+ * router in their first launch.  Whole layer, GEMV -> GEMM us, for hidden x
+ * intermediate size, routed experts, experts per token (+ shared):
+ *   2048 x 1408, 64, 6 + 2   5 tokens 120 -> 115, 6: 138 -> 131, 8: 177 -> 154
+ *   2048 x 1536, 64, 4 + 1   5 tokens (120 MB saved) 93 -> 95, 6 (159 MB) 106 -> 98
+ *   2048 x 1408, 16, 2 + 1   5 tokens (108 MB) 62 -> 63, 6 (141 MB) 69 -> 64
+ *   4096 x 14336, 8, 2       5 tokens 648 -> 390
+ *   1024 x 512, 8, 2 + 1     8 tokens (50 MB) 32 -> 35, 9: 50 -> 35
+ *   256 x 128, 16, 4 + 2     8 tokens 19 -> 27, 9: 37 -> 27
+ *   2048 x 512, 256, 8 + 1   8 tokens 176 -> 211, 9: 277 -> 227 */
 #ifndef MM_BF16_MM_MIN_T
 #define MM_BF16_MM_MIN_T 5
+#define MM_BF16_MM_SAVED 128e6
 #endif
+#define MM_BF16_NT_MAX 8          /* tokens per pass of the GEMV stages */
 /* Rows of one pass, and bytes of its workspace: 180 KB per row at DeepSeek-V2-Lite's
  * sizes (370 MB), 750 KB at a hidden size of 7,168 with 8 experts of 2,048 per token. */
 #define MM_BF16_MM_T_CHUNK 2048

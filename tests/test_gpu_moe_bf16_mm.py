@@ -54,7 +54,7 @@ def run(H, E, K, I, NS, T, hot=False, scale=1.0, seed=0, chunk=None):
     return out
 
 
-@pytest.mark.parametrize("T", [5, 6, 16, 17, 33, 64, 65, 131])
+@pytest.mark.parametrize("T", [5, 6, 9, 16, 17, 33, 64, 65, 131])
 @pytest.mark.parametrize("hot", [False, True])
 def test_row_tiles(T, hot):
     run(256, 8, 2, 128, 2, T, hot, seed=T)
@@ -64,6 +64,25 @@ def test_row_tiles(T, hot):
                                           (256, 300, 8, 64, 1, 37), (128, 160, 4, 64, 3, 90), (64, 2, 2, 200, 2, 300)])
 def test_shapes(H, E, K, I, NS, T):
     run(H, E, K, I, NS, T, seed=H + I)
+
+
+@pytest.mark.parametrize("H,E,K,I,NS,T,grouped", [
+    (256, 16, 4, 128, 2, 8, 0), (256, 16, 4, 128, 2, 9, 1),              # the GEMV stages' one pass, their second
+    (1024, 4, 2, 2048, 0, 7, 0), (1024, 4, 2, 2048, 0, 8, 1),            # 126 and 151 MB of weights not read again
+    (2048, 4, 4, 2048, 0, 4, 0), (2048, 4, 4, 2048, 0, 5, 1),            # 4 tokens stay with the GEMV
+    (512, 65, 8, 2048, 4, 8, 0)])                                        # more than 64 experts
+def test_rule(H, E, K, I, NS, T, grouped):
+    w, x = synth.moe_layer(940, H, E, I, NS), synth.activations(941, T, H)
+    with mlamoe.Context(0) as ctx:
+        ctx.moe_init(H, E, NS, K, I)
+        ctx.moe_load_layer(0, w, mlamoe.MM_LOAD_BF16)
+        ctx.prof_enable(True)
+        out, idx, wt, _ = ctx.moe_forward(0, x)
+        ran = ctx.prof_query("mm_bf16_rows")[1]
+        ctx.prof_enable(False)
+    ref = ref64(w, x, idx, wt, NS)
+    assert np.linalg.norm(out - ref) < TOL * np.linalg.norm(ref)
+    assert ran == grouped
 
 
 def test_passes_agree():
