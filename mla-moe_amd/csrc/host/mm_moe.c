@@ -919,8 +919,10 @@ static int forward_int8(mm_ctx *c, const mm_moe_layer *L, int T, const float *xn
     /* decode-shaped GEMMs stage a 16-row A tile (16 * K bytes) and a row list
      * (T ints) in LDS; shapes beyond 64 KB of it take the tiled GEMMs */
     const size_t lds_dec = 16 * (H > (I > S ? I : S) ? H : (I > S ? I : S)) + 4 * (size_t)T;
+    size_t rows_min = MM_I8_TILED_ROWS * E + MM_I8_TILED_BYTES / (3 * I * H);
+    if (rows_min > MM_I8_TILED_MAX * E) rows_min = MM_I8_TILED_MAX * E;
     const int tiled = lds_dec > 65536 || (c->i8_tiled_min_t >= 0 ? T >= c->i8_tiled_min_t
-                                                                 : T >= MM_I8_TILED_T || R >= MM_I8_TILED_ROWS * E);
+                                                                 : T >= MM_I8_TILED_T || R >= rows_min);
     /* which SwiGLU: a call that the rows per expert alone made tiled has the
      * decode-shaped GEMM's */
     const int gu = lds_dec <= 65536 && c->i8_tiled_min_t < 0 && T < MM_I8_TILED_T ? 2 : 1;

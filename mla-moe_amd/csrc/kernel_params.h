@@ -322,20 +322,33 @@ typedef struct {
 #define MM_I8S_RT 4                /* row-tile blocks per shared-expert column group */
 #define MM_I8S_XCD 8               /* blocks are dealt to XCDs round robin */
 
-/* Tiled GEMMs from MM_I8_TILED_T tokens on, or from MM_I8_TILED_ROWS rows per
- * expert on average.  A decode-shaped block streams its expert's weights once
- * per 16 rows, so its time doubles soon after the experts' row counts pass 16;
- * a tile reads them once per 128 rows but costs more to fill.  Whole layer
- * (DeepSeek-V2-Lite: 64 experts, 6 per token, even routing), decode-shaped ->
- * tiled: 96 tokens (9 rows) 142 -> 166 us, 112 tokens 152 -> 168, 160 tokens
- * (15 rows) 210 -> 169, 255 tokens 281 -> 177; Zipf-skewed routing crosses
- * below 56 tokens, which the host cannot know (it does not see the routing).
- * Calls that only the second bound sends here keep the decode-shaped GEMM's
- * SwiGLU (gu = 2), so both forms give the same bits: with the hardware
- * exponential a few hidden values round to the next int8 (181 tokens: error
- * against 64 bits 1.9e-7 -> 2.1e-5; time 153 us with it, 156 without). */
+/* Tiled GEMMs from MM_I8_TILED_T tokens on, and below that from MM_I8_TILED_ROWS
+ * rows per expert on average plus MM_I8_TILED_BYTES of an expert's weights for
+ * the rows beyond (all experts together), at most MM_I8_TILED_MAX rows per
+ * expert.  A decode-shaped block streams its expert's weights once per 16 rows,
+ * so the calls get longer soon after the row counts pass 12 (some experts have
+ * more), by the bytes of the extra passes; a tile reads them once per 128 rows
+ * but costs some 15 (small layers) to 40 us more to fill.  Small layers' extra
+ * passes come out of the caches and cost little: there the tiles win late.
+ * Whole layer with even routing, decode-shaped -> tiled us; hidden x
+ * intermediate size, routed experts, experts per token, weights of an expert,
+ * rows per expert at which the rule turns:
+ *   2048 x 1408, 64, 6, 8.7 MB, 12.9   128 tokens 157 -> 168, 136: 170 -> 166, 160: 191 -> 167
+ *   2048 x 1536, 64, 4, 9.4 MB, 12.8   192 tokens 170 -> 175, 208: 191 -> 177
+ *   2048 x 1024, 32, 4, 6.3 MB, 14.4   104 tokens 79 -> 70, 128: 91 -> 71
+ *   1024 x 512, 64, 6, 1.6 MB, 16.8    160 tokens 64 -> 66, 184: 70 -> 67
+ *   1024 x 512, 8, 2, 1.6 MB, 50       128 tokens 41 -> 46, 176: 48 -> 46, 224: 58 -> 47
+ *   256 x 128, 16, 4, 0.1 MB, 56       48 tokens 25 -> 35, 208: 37 -> 37, 224: 40 -> 37
+ * Skewed routing crosses earlier (Zipf, the first of these: below 56 tokens),
+ * which the host cannot know: it does not see the routing.
+ * Calls that only the rows send here keep the decode-shaped GEMM's SwiGLU
+ * (gu = 2), so both forms give the same bits: with the hardware exponential a
+ * few hidden values round to the next int8 (181 tokens: error against 64 bits
+ * 1.9e-7 -> 2.1e-5; time 153 us with it, 156 without). */
 #define MM_I8_TILED_T 256
 #define MM_I8_TILED_ROWS 12
+#define MM_I8_TILED_BYTES 480000000
+#define MM_I8_TILED_MAX 56
 
 /* Grouped int8 GEMM for prefill sizes (mm_i8_gemm_bt, gemm_i8.hip): block
  * tiles of 128 rows x 16 B fragments over the routed experts' row lists (or
