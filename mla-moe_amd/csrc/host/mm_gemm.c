@@ -166,18 +166,22 @@ int mm_gemm_bf16_add_rmsnorm_hl(mm_ctx *c, float *x, const uint16_t *ahl, const 
 static int gemm_bf16_rows(mm_ctx *c, float *y, const uint16_t *xh, const uint16_t *xl,
                           const uint16_t *w, int d_out, float *y1, const uint16_t *w1, int d1, int n_in,
                           int kp, int T, int split, int acc) {
-    /* block tile columns: the widest of 128, 64, 32 that still gives 192
-     * tiles (most of the 256 CUs), else 32 -- the projections of this path
-     * have too few 128 x 128 tiles to fill the machine (measured per width) */
     int span = MM_GB_BM;   /* rows (or columns) of a tile, by their bytes */
     while ((size_t)span * (size_t)kp * 2 > MM_GB_SPAN) span /= 2;
     const size_t nby = ((size_t)T + span - 1) / span;
-    int bn = 32;
-    for (int cw = 128; cw >= 64; cw /= 2)
-        if ((((size_t)d_out + cw - 1) / cw + ((size_t)d1 + cw - 1) / cw) * nby >= 192) {
-            bn = cw;
-            break;
-        }
+    /* block tile columns: the width with the shortest rounds of the 256 CUs in
+     * all.  A round of 128, 64 or 32 columns takes about 6 : 4 : 3 (10,944
+     * columns, 2,048 inputs: 400 rows in two rounds of 128 columns 58 us in
+     * split mode, 39 truncated; 200 rows in two of 64 39 and 31; 65 rows in two
+     * of 32 29 and 22); of equal ones the widest, which reads x fewest times. */
+    int bn = 0;
+    for (size_t cw = 128, wt = 6, best = 0; cw >= 32; cw /= 2, wt = cw == 64 ? 4 : 3) {
+        const size_t tiles = (((size_t)d_out + cw - 1) / cw + ((size_t)d1 + cw - 1) / cw) * nby;
+        const size_t cost = (tiles + 255) / 256 * wt;
+        if (bn && cost >= best) continue;
+        best = cost;
+        bn = (int)cw;
+    }
     const int cols = bn < span ? bn : span;
     const size_t nb0 = ((size_t)d_out + cols - 1) / cols, nbx = nb0 + ((size_t)d1 + cols - 1) / cols;
     /* the XCDs' rectangle of tiles: fewest rounds of an XCD's 32 CUs, then

@@ -44,6 +44,18 @@ def test_tiles_exact(ctx, T, d, n, flags):
     assert np.array_equal(ctx.matmul(x, wb, flags | mlamoe.MM_MATMUL_ACCUMULATE, y0=y0), want + y0)
 
 
+@pytest.mark.parametrize("T,d,n,bn", [(65, 8200, 72, 64),        # 129 tiles of 64 columns: one round, 257 of 32 two
+                                      (100, 8192, 72, 32),       # 256 of 32: one round
+                                      (200, 16400, 72, 128),     # 258 of 128: two rounds, 514 of 64 three
+                                      (1920, 570, 72, 64)])
+def test_column_widths(ctx, T, d, n, bn):
+    """Shapes either side of a whole round of tiles per width; exact."""
+    rng = np.random.default_rng(d)
+    x, w = ints(rng, (T, n)), ints(rng, (d, n))
+    print(f"widths T={T} d={d} n={n}: {bn} columns", flush=True)
+    assert np.array_equal(ctx.matmul(x, synth.bf16_from_f32(w), mlamoe.MM_MATMUL_X_BF16), x @ w.T)
+
+
 def test_unaligned_output(ctx):
     T, d, n = 140, 132, 128
     rng = np.random.default_rng(9)
