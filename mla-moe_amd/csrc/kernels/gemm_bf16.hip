@@ -270,25 +270,44 @@ __device__ __forceinline__ void gemm_block(const mm_gemm_bf16_args &a, uint8_t *
 
     /* lane l holds row l % 32 and, in registers 4 g + i, columns 8 g + 4 (l /
      * 32) + i of each 32 x 32 tile (the weights are the first operand).  With
-     * accumulate, a row tile's old outputs are all loaded (clamped addresses,
-     * unconditionally) before any is added. */
+     * accumulate, the wave's old outputs are all loaded (clamped addresses,
+     * unconditionally) before any is added, four at a time in a tile of whole
+     * columns (2,048 rows, accumulated: 64 x 64 7.9 us, 4096 x 512 38; one value
+     * at a time, a row tile after the other, 9.3 and 46). */
     float *y = second ? a.y1 : a.y;
-    const bool acc_old = a.accumulate && !second;
     const int mend = m0 + mrows, nend = n0 + ncols;
+    auto row_of = [&](int t) { return y + (size_t)min(m0 + 64 * wm + 32 * t + c32, mend - 1) * d_out; };
+    if (a.accumulate && !second) {   /* uniform */
+        f32x16 prev[2][WT];
+        if (n0 + cw + 32 * WT <= nend) {
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int j = 0; j < WT; j++)
+#pragma unroll
+                    for (int g = 0; g < 4; g++) {
+                        const f32x4 v = *(const f32x4_a4 *)(row_of(t) + n0 + cw + 32 * j + 8 * g + 4 * hi);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) prev[t][j][4 * g + i] = v[i];
+                    }
+        } else {
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int j = 0; j < WT; j++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++)
+                        prev[t][j][i] = row_of(t)[min(n0 + cw + 32 * j + 8 * (i >> 2) + 4 * hi + (i & 3), nend - 1)];
+        }
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int j = 0; j < WT; j++) sum[t][j] = prev[t][j] + sum[t][j];
+    }
 #pragma unroll
     for (int t = 0; t < 2; t++) {
         const int m = m0 + 64 * wm + 32 * t + c32;
-        float *row = y + (size_t)min(m, mend - 1) * d_out;
-        if (acc_old) {   /* uniform */
-            f32x16 prev[WT];
-#pragma unroll
-            for (int j = 0; j < WT; j++)
-#pragma unroll
-                for (int i = 0; i < 16; i++)
-                    prev[j][i] = row[min(n0 + cw + 32 * j + 8 * (i >> 2) + 4 * hi + (i & 3), nend - 1)];
-#pragma unroll
-            for (int j = 0; j < WT; j++) sum[t][j] = prev[j] + sum[t][j];
-        }
+        float *row = row_of(t);
 #pragma unroll
         for (int j = 0; j < WT; j++)
 #pragma unroll
