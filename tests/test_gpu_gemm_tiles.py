@@ -31,7 +31,8 @@ def ctx():
 @pytest.mark.parametrize("T,d,n", [
     (65, 31, 64), (128, 32, 72), (129, 33, 200), (300, 100, 136),       # 32-column tiles
     (513, 2501, 64), (1100, 1730, 128), (640, 4097, 264),              # 64 and 128 columns
-    (2047, 2048, 192), (2100, 3648, 320), (37, 70, 264), (9000, 65, 576)])
+    (2047, 2048, 192), (2100, 3648, 320), (37, 70, 264), (9000, 65, 576),
+    (70, 40, 1096), (1920, 570, 1096), (2000, 2000, 1160)])           # 32, 64, 128 columns: every ring wraps, sums move
 @pytest.mark.parametrize("flags", [0, mlamoe.MM_MATMUL_X_BF16])
 def test_tiles_exact(ctx, T, d, n, flags):
     rng = np.random.default_rng(T + d + n)

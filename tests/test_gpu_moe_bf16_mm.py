@@ -61,7 +61,9 @@ def test_row_tiles(T, hot):
 
 
 @pytest.mark.parametrize("H,E,K,I,NS,T", [(264, 4, 2, 72, 1, 70), (72, 3, 1, 8, 0, 40), (1032, 6, 3, 136, 1, 9),
-                                          (256, 300, 8, 64, 1, 37), (128, 160, 4, 64, 3, 90), (64, 2, 2, 200, 2, 300)])
+                                          (256, 300, 8, 64, 1, 37), (128, 160, 4, 64, 3, 90), (64, 2, 2, 200, 2, 300),
+                                          # 16, 32 and 64 rows per tile where the sums move every 256 values
+                                          (1032, 8, 2, 520, 1, 30), (1032, 8, 2, 520, 1, 64), (1032, 8, 2, 520, 1, 131)])
 def test_shapes(H, E, K, I, NS, T):
     run(H, E, K, I, NS, T, seed=H + I)
 

@@ -1,5 +1,5 @@
 """Prefill attention in the expanded form (keys and values per head, the rows
-of a prompt in 128-row tiles): prompts at the edges of its tiles, several
+of a prompt in 64-row tiles): prompts at the edges of its tiles, several
 prompts of unequal length in one step, a chunk after earlier positions, and
 decode rows beside them, against the absorbed form of the same engine.
 
@@ -27,46 +27,72 @@ def model():
                        c["dense_inter"], c["E"], c["I"], c["n_shared"], c["vocab"])
 
 
-def logits(model, steps, monkeypatch, expand_min):
-    """Each step: a list of (slot, first position, rows).  All rows' logits."""
+def logits(model, steps, monkeypatch, expand_min, cfg=CFG):
+    """Each step: a list of (slot, first position, rows).  All rows' logits,
+    and each step's launches of the expanded and the absorbed attention per
+    layer."""
     monkeypatch.setenv("MLAMOE_MLA_EXPAND_MIN", str(expand_min))
     rng = np.random.default_rng(5)
     toks = rng.integers(0, CFG["vocab"], (8, 2048)).astype(np.int32)
-    out = []
+    out, forms = [], []
     with mlamoe.Context(0) as ctx:
-        eng = Engine.from_host(ctx, CFG, model, mlamoe.rope_inv_freq(64, 10000.0), max_batch=8, max_seq=1200,
+        eng = Engine.from_host(ctx, cfg, model, mlamoe.rope_inv_freq(64, 10000.0), max_batch=8, max_seq=1200,
                                max_rows=2048)
         try:
             for st in steps:
+                ctx.prof_reset()
+                ctx.prof_enable(True)
                 rows = [(s, p0 + i) for s, p0, n in st for i in range(n)]
                 sl, ps = (np.array(a, np.int32) for a in zip(*rows))
                 _, lg = eng.step_rows(sl, toks[sl, ps], ps, np.arange(len(rows)), want_logits=True)
                 out.append(lg)
+                ctx.prof_enable(False)
+                n = [ctx.prof_query(k)[1] // cfg["n_layers"]
+                     for k in ("mm_mla_attn_expanded", "mm_mla_attn", "mm_mla_attn_rows")]
+                forms.append((n[0], n[1] + n[2]))
         finally:
             eng.close()
-    return np.concatenate(out).astype(np.float64)
+    return np.concatenate(out).astype(np.float64), forms
 
 
-@pytest.mark.parametrize("steps", [
-    [[(0, 0, 128)]], [[(0, 0, 129)]], [[(3, 0, 161)]], [[(0, 0, 65)]], [[(1, 0, 1023)]],
-    [[(0, 0, 300), (1, 0, 50), (2, 0, 128), (5, 0, 255)]],                  # unequal prompts (50: absorbed)
-    [[(0, 0, 37)], [(0, 37, 200), (1, 0, 130)], [(0, 237, 1), (1, 130, 1), (2, 0, 140)]],   # chunks, decode rows
-    [[(0, 0, 31)], [(0, 31, 66)], [(0, 97, 513)]],
-    [[(0, 0, 1000), (1, 0, 1000)], [(0, 1000, 100), (1, 1000, 150)]],
-], ids=lambda s: "-".join("+".join(str(n) for _, _, n in st) for st in s))
-def test_expanded_agrees_with_absorbed(model, monkeypatch, steps):
-    a = logits(model, steps, monkeypatch, 65)
-    b = logits(model, steps, monkeypatch, 0)
+# with each step's launches per layer: expanded, absorbed
+@pytest.mark.parametrize("steps,want", [
+    ([[(0, 0, 128)]], [(1, 0)]), ([[(0, 0, 129)]], [(1, 0)]), ([[(3, 0, 161)]], [(1, 0)]), ([[(0, 0, 65)]], [(1, 0)]),
+    ([[(1, 0, 1023)]], [(1, 0)]),
+    ([[(0, 0, 300), (1, 0, 50), (2, 0, 128), (5, 0, 255)]], [(1, 1)]),      # unequal prompts (50: absorbed)
+    # chunks, decode rows
+    ([[(0, 0, 37)], [(0, 37, 200), (1, 0, 130)], [(0, 237, 1), (1, 130, 1), (2, 0, 140)]], [(0, 1), (1, 0), (1, 1)]),
+    ([[(0, 0, 31)], [(0, 31, 66)], [(0, 97, 513)]], [(0, 1), (1, 0), (1, 0)]),
+    ([[(0, 0, 1000), (1, 0, 1000)], [(0, 1000, 100), (1, 1000, 150)]], [(1, 0), (1, 0)]),
+], ids=lambda v: "-".join("+".join(str(n) for _, _, n in st) if isinstance(st, list) else "%dx%d" % st for st in v))
+def test_expanded_agrees_with_absorbed(model, monkeypatch, steps, want):
+    a, forms = logits(model, steps, monkeypatch, 65)
+    b, absorbed = logits(model, steps, monkeypatch, 0)
+    assert forms == want and not any(e for e, _ in absorbed)
     err = np.linalg.norm(a - b) / np.linalg.norm(b)
     worst = np.max(np.linalg.norm(a - b, axis=1) / np.linalg.norm(b, axis=1))
     print(f"{steps}: {err:.2e}, worst row {worst:.2e}", flush=True)
     assert err < 2e-4 and worst < 2e-3
-    assert err > 0                       # another form did run
+
+
+def test_more_tiles_than_compute_units(monkeypatch):
+    """16 heads: 16 row tiles give every CU one block, and the host puts the
+    next 16 in reverse order.  18, 30 and 33 tiles: every row once."""
+    c = dict(CFG, NH=16)
+    m = synth.model(4323, c["n_layers"], c["first_dense"], c["H"], c["NH"], c["QKN"], c["QKR"], c["KVL"], c["VHD"],
+                    c["dense_inter"], c["E"], c["I"], c["n_shared"], c["vocab"])
+    for steps in ([[(0, 0, 1150), (1, 0, 898)]], [[(0, 0, 640), (1, 0, 640), (2, 0, 640)]], [[(0, 0, 1089)]]):
+        a, forms = logits(m, steps, monkeypatch, 65, c)
+        b, _ = logits(m, steps, monkeypatch, 0, c)
+        assert forms == [(1, 0)]
+        worst = np.max(np.linalg.norm(a - b, axis=1) / np.linalg.norm(b, axis=1))
+        assert np.linalg.norm(a - b) < 2e-4 * np.linalg.norm(b) and worst < 2e-3
 
 
 def test_expanded_against_oracle(model, monkeypatch, oracle):
     """Every position of a 150-token prompt against the reference's forward."""
-    got = logits(model, [[(0, 0, 150)]], monkeypatch, 128)
+    got, forms = logits(model, [[(0, 0, 150)]], monkeypatch, 128)
+    assert forms == [(1, 0)]
     toks = np.random.default_rng(5).integers(0, CFG["vocab"], (8, 2048)).astype(np.int32)[0, :150]
     ref = oracle.model_logits(CFG, model, toks, mlamoe.rope_inv_freq(64, 10000.0))
     err = np.max(np.abs(got - ref), axis=1) / np.max(np.abs(ref), axis=1)
@@ -76,11 +102,13 @@ def test_expanded_against_oracle(model, monkeypatch, oracle):
 
 def test_scratch_cap_falls_back(model, monkeypatch):
     """Prompts whose expanded keys do not fit the attention scratch cap take
-    the absorbed form: here the second of two."""
-    monkeypatch.setenv("MLAMOE_MLA_PART_MAX", str(40 * 4 * 32768))     # 40 blocks of 4 heads
+    the absorbed form: neither of two, the second, the first, both."""
     steps = [[(0, 0, 1000), (1, 0, 600)]]
-    a = logits(model, steps, monkeypatch, 128)
-    b = logits(model, steps, monkeypatch, 0)
+    for blocks, want in ((32 + 19, (1, 0)), (40, (1, 1)), (31, (1, 1)), (18, (0, 1))):     # 32 keys of 4 heads each
+        monkeypatch.setenv("MLAMOE_MLA_PART_MAX", str(blocks * 4 * 32768))
+        a, forms = logits(model, steps, monkeypatch, 128)
+        assert [(e, min(n, 1)) for e, n in forms] == [want]       # (absorbed rows go in groups within the cap)
+    b, _ = logits(model, steps, monkeypatch, 0)
     assert np.linalg.norm(a - b) < 2e-4 * np.linalg.norm(b)
 
 
