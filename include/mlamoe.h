@@ -194,10 +194,10 @@ MM_API int mm_moe_forward_dev(mm_ctx *ctx, int layer, int T, const float *xn, fl
  * Same arguments, kernels and results; the call's workspace is a static
  * device array of MM_NOALLOC_SCRATCH_BYTES per device (32 MiB: e.g. up to
  * ~280 tokens of a DeepSeek-V2-Lite int8 layer, 64 for the bench's decode
- * batch) instead of the context's growable buffer.  A call that would need
- * more fails with MM_ERR_UNSUPPORTED before launching anything.  Every call
- * on a device shares that
- * device's array: calls that overlap on one device (two streams, two host
+ * batch) instead of the context's growable buffer.  An int8 or dense call
+ * that would need more fails with MM_ERR_UNSUPPORTED before launching anything;
+ * a bf16 MoE call runs in passes of as many tokens as the array holds.  Every
+ * call on a device shares that device's array: calls that overlap on one device (two streams, two host
  * threads) race.  While per-kernel profiling is on (mm_prof_enable) it
  * returns MM_ERR_STATE: the profiler's records are host allocations. */
 #define MM_NOALLOC_SCRATCH_BYTES (32u << 20)

@@ -51,8 +51,9 @@ int mm_moe_init(mm_ctx *c, const mm_moe_config *cfg, int n_layers) {
         return mm_fail(MM_ERR_UNSUPPORTED, "mm_moe_init: hidden and moe_inter must be multiples of 8");
     int st = mm_set_device(c);
     if (st) return st;
-    /* per-expert counters of the tiled int8 path, or per-token counters of
-     * the bf16 router + shared launch (RSH_TMAX tokens): zero between calls */
+    /* per-expert counters of the tiled int8 and the grouped bf16 GEMMs, or
+     * per-token counters of the bf16 router + shared launch (RSH_TMAX tokens):
+     * zero between calls */
     const size_t ncnt = (size_t)E * MM_CNT_STRIDE;   /* >= RSH_TMAX */
     MM_HIP(hipMalloc((void **)&c->moe_cnt, ncnt * sizeof(int32_t)));
     MM_HIP(hipMemsetAsync(c->moe_cnt, 0, ncnt * sizeof(int32_t), c->stream));
@@ -611,7 +612,11 @@ static int bf16_mm_pass(mm_ctx *c, const mm_moe_layer *L, int T, const float *xn
         return clear_counters(c, st);
     /* rows per tile by the mean rows of an expert (R routes over E): fewer
      * rows leave LDS for a deeper weight ring, more read an expert's weights
-     * fewer times */
+     * fewer times.  Whole layer in us by 16, 32 and 64 rows per tile:
+     *   2048 x 1408, 64 experts, 6 + 2   6 rows 243, 241, 279; 9: 250, 260, 284;
+     *       12: 279, 275, 295; 24: 389, 319, 345; 30: 462, 397, 360
+     *   2048 x 1536, 64 experts, 4 + 1   8 rows 255, 262, 297; 12: 283, 273, 309;
+     *       20: 403, 332, 342; 25: 424, 362, 352 */
     const size_t mean = ((size_t)R + E - 1) / E;
     const int bm = mean <= 8 ? 0 : mean <= 24 ? 1 : 2;
     static const mm_kernel_id kgu[3] = {K_BF16_GU_16, K_BF16_GU_32, K_BF16_GU_64};

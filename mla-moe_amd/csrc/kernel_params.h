@@ -19,8 +19,9 @@
  * 3: 33 against 39 us; 16 per block leave half the CUs idle, 50 us) */
 #define MM_ROUTER_WAVES_LOGITS 8
 
-/* Logits-only router with one token per block (mm_router_pc): used for
- * E <= 64, H % 8 == 0 and T up to this many tokens. */
+/* Router with one token per block: E <= 64, H % 8 == 0 and T up to this many
+ * tokens.  mm_router_pc_split for logits alone; mm_router_pc, with the top-k,
+ * for 5 to 8 tokens of a pass of the bf16 GEMV stages. */
 #define MM_ROUTER_PC_TMAX 256
 #ifndef MM_ROUTER_PC_EB
 #define MM_ROUTER_PC_EB 16        /* experts per block of the logits-only product/chain router */
@@ -100,8 +101,8 @@ typedef struct {
 #define MM_BF16_MM_SAVED 128e6
 #endif
 #define MM_BF16_NT_MAX 8          /* tokens per pass of the GEMV stages */
-/* Rows of one pass, and bytes of its workspace: 180 KB per row at DeepSeek-V2-Lite's
- * sizes (370 MB), 750 KB at a hidden size of 7,168 with 8 experts of 2,048 per token. */
+/* Rows of one pass, and bytes of its workspace: 212 KB per row at DeepSeek-V2-Lite's
+ * sizes (433 MB), 750 KB at a hidden size of 7,168 with 8 experts of 2,048 per token. */
 #define MM_BF16_MM_T_CHUNK 2048
 #define MM_BF16_MM_WS ((size_t)1 << 30)
 #define MM_BF16_MM_GRID 256       /* persistent grid: one block per CU */
@@ -271,8 +272,8 @@ typedef struct {
 
 /* out[t] (=|+=) sum_r w[t,r] * y[t*K + r] + ys[t] (with yrow, route t*K + r's
  * row of y is yrow[t*K + r]); clears the E counters
- * cnt[e * MM_CNT_STRIDE] when cnt is given (the tiled path's per-expert
- * counters, read by then). */
+ * cnt[e * MM_CNT_STRIDE] when cnt is given (the per-expert counters of the
+ * tiled int8 and the grouped bf16 GEMMs, read by then). */
 typedef struct {
     const float *y, *ys;
     const float *topk_w;
@@ -490,9 +491,10 @@ typedef struct {
 /* A step's rows of one sequence are attended in the expanded form from
  * MM_MLA_EXPAND_MIN rows on, and from one row per MM_MLA_EXPAND_KEYS keys:
  * fewer do not pay for expanding the keys, and are too few blocks for long
- * chains (4-layer step, absorbed and expanded: 65 rows 1035 and 1005 us, after
- * 1,000 positions 1150 and 1147, after 4,000 1316 and 1586; 192 rows after
- * 4,000 1957 and 1990, 256 rows 2170 and 1898, 512 rows 2946 and 2122). */
+ * chains (4-layer step, absorbed and expanded: 65 rows 982 and 942 us, after
+ * 1,000 positions 1104 and 1079, after 1,235 (the line) 1111 and 1128, after
+ * 4,000 1275 and 1534; 192 rows after 3,648 (the line) 1742 and 1667, after
+ * 4,000 1748 and 1740; 256 after 4,000 2119 and 1829, 512 2909 and 2017). */
 #define MM_MLA_EXPAND_MIN 65
 #define MM_MLA_EXPAND_KEYS 20
 #define MM_MLA_XNS 2              /* chunks of latent values in an expanding block's ring */

@@ -61,8 +61,8 @@ extern "C" __global__ __launch_bounds__(256) void mm_cvt_bf16(mm_cvt_bf16_args a
  * reads' round trip and the MFMAs of a chunk added up (split mode, 2,048
  * rows: 2,048 x 2,048 49 us, 2,048 x 10,944 209, 10,944 x 2,048 270; now 32,
  * 153 and 178: 1,030-1,200 TFLOP/s of MFMAs, what a library product of 8,192
- * cubed reaches here; 512 truncated rows through the four projections 59 us
- * -> 39).  Its parts alone, 2,048 x 10,944: the loads 108 us (48 KB per chunk
+ * cubed reaches here; 512 truncated rows through the four projections 58 us
+ * -> 53).  Its parts alone, 2,048 x 10,944: the loads 108 us (48 KB per chunk
  * and CU: 20 TB/s out of L2), the MFMAs 100, both 153: they share the LDS.
  *
  * GB_FLUSH: the accumulators are added to a second set every 512 values of

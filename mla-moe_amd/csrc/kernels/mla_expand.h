@@ -9,7 +9,8 @@
  * and the absorbed queries and W_UV products of every row go.  The price is
  * one pass over the latent cache per layer (mm_mla_expand: 2 x 128 x 512
  * products per key and head, both operands bf16, no pairs), so it pays from
- * about a hundred rows per key range on.
+ * 65 rows on, and from one row per 20 keys (MM_MLA_EXPAND_MIN,
+ * MM_MLA_EXPAND_KEYS).
  *
  * All four products of two pairs are kept: without lo * lo the error against
  * 64 bits is 15% above the absorbed form's (emulated, 700 random keys: 4.9e-6
