@@ -415,6 +415,10 @@ static int engine_run(mm_engine *e, int R, int n_want, int32_t *next, float *log
     step_plan p;
     if (!(st = plan_step(e, R, &p))) st = run_planned(e, R, n_want, next, logits, &p);
     free(p.abs);
+    /* a step that failed on its way has copies of h_io and xt_h queued, which
+     * the next step fills anew: tile tables of one step must not reach another's
+     * launches (a step that ends waits by itself) */
+    if (st) (void)hipStreamSynchronize(c->stream);
     return st;
 }
 

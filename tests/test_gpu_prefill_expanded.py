@@ -171,3 +171,24 @@ def test_row_that_is_not_finite(model, first, n, bad, value):
             eng.close()
     assert np.array_equal(out[0][:bad], out[1][:bad])
     assert np.isfinite(out[0]).all() and np.isnan(out[1][bad:]).all()
+
+
+def test_step_after_one_that_failed(model, monkeypatch):
+    """A step that fails on its way (no room for its absorbed scratch either)
+    leaves nothing queued that the next one's tables could reach."""
+    toks = np.random.default_rng(8).integers(0, CFG["vocab"], 2048).astype(np.int32)
+    out = []
+    for limit in (None, 8 << 20):                  # 2,048 rows: 8 MB of expanded keys and their bits, 33 MB absorbed
+        if limit:
+            monkeypatch.setenv("MLAMOE_WS_MAX", str(limit))
+        with mlamoe.Context(0) as ctx:
+            eng = Engine.from_host(ctx, CFG, model, mlamoe.rope_inv_freq(64, 10000.0), max_batch=2, max_seq=2048,
+                                   init_seq=2048, max_rows=2048)
+            try:
+                for _ in range(3 if limit else 0):
+                    with pytest.raises(mlamoe.MMError, match="workspace"):
+                        eng.step_rows(np.zeros(2048), toks, np.arange(2048), [])
+                out.append(eng.step_rows(np.ones(130), toks[:130], np.arange(130), np.arange(130), want_logits=True)[1])
+            finally:
+                eng.close()
+    assert np.array_equal(out[0], out[1])
