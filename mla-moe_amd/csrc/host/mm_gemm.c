@@ -169,32 +169,32 @@ static int gemm_bf16_rows(mm_ctx *c, float *y, const uint16_t *xh, const uint16_
     int span = MM_GB_BM;   /* rows (or columns) of a tile, by their bytes */
     while ((size_t)span * (size_t)kp * 2 > MM_GB_SPAN) span /= 2;
     const size_t nby = ((size_t)T + span - 1) / span;
-    /* block tile columns: the width with the shortest rounds of the 256 CUs in
-     * all.  A round of 128, 64 or 32 columns takes about 6 : 4 : 3 (10,944
+    /* Block tile columns, and the XCDs' rectangle of tiles (xr down, 8 / xr
+     * across): the shortest rounds of an XCD's 32 CUs in all, a CU holding one
+     * block.  A round of 128, 64 or 32 columns takes about 6 : 4 : 3 (10,944
      * columns, 2,048 inputs: 400 rows in two rounds of 128 columns 58 us in
      * split mode, 39 truncated; 200 rows in two of 64 39 and 31; 65 rows in two
-     * of 32 29 and 22); of equal ones the widest, which reads x fewest times. */
-    int bn = 0;
-    for (size_t cw = 128, wt = 6, best = 0; cw >= 32; cw /= 2, wt = cw == 64 ? 4 : 3) {
-        const size_t tiles = (((size_t)d_out + cw - 1) / cw + ((size_t)d1 + cw - 1) / cw) * nby;
-        const size_t cost = (tiles + 255) / 256 * wt;
-        if (bn && cost >= best) continue;
-        best = cost;
-        bn = (int)cw;
-    }
-    const int cols = bn < span ? bn : span;
-    const size_t nb0 = ((size_t)d_out + cols - 1) / cols, nbx = nb0 + ((size_t)d1 + cols - 1) / cols;
-    /* the XCDs' rectangle of tiles: fewest rounds of an XCD's 32 CUs, then
-     * fewest operand rows read into an XCD's L2 (x rows count once per plane) */
-    size_t best = 0, blocks = 0;
-    int xr = 1;
-    for (int r = 1; r <= 8; r *= 2) {
-        const size_t pr = (nby + r - 1) / r, pc = (nbx + 8 / r - 1) / (8 / r);
-        const size_t cost = ((pr * pc + 31) / 32 << 32) + pr * MM_GB_BM * (split ? 2 : 1) + pc * bn;
-        if (r > 1 && cost >= best) continue;
-        best = cost;
-        xr = r;
-        blocks = 8 * pr * pc;
+     * of 32 29 and 22).  Of equal ones the widest, which reads x fewest times,
+     * then the fewest operand rows read into an XCD's L2 (x rows count once per
+     * plane).  649 x 1,327 x 152, truncated: 252 tiles of 32 columns, but 33 at
+     * least in some XCD: 12.3 us, 64 columns in one round 8.8. */
+    int bn = 0, cols = 0, xr = 1;
+    size_t best = 0, least = 0, nb0 = 0, blocks = 0;
+    for (int cw = 128, wt = 6; cw >= 32; cw /= 2, wt = cw == 64 ? 4 : 3) {
+        const int cu = cw < span ? cw : span;
+        const size_t n0 = ((size_t)d_out + cu - 1) / cu, nbx = n0 + ((size_t)d1 + cu - 1) / cu;
+        for (int r = 1; r <= 8; r *= 2) {
+            const size_t pr = (nby + r - 1) / r, pc = (nbx + 8 / r - 1) / (8 / r);
+            const size_t cost = (pr * pc + 31) / 32 * wt, rows = pr * span * (split ? 2 : 1) + pc * cu;
+            if (bn && (cost > best || (cost == best && (cw != bn || rows >= least)))) continue;
+            best = cost;
+            least = rows;
+            bn = cw;
+            cols = cu;
+            xr = r;
+            nb0 = n0;
+            blocks = 8 * pr * pc;
+        }
     }
     mm_gemm_bf16_args a = {xh, xl, w, y, T, d_out, n_in, kp, split, acc, bn, (int)nb0, d1 ? w1 : NULL, y1, d1, xr,
                            span, cols};
