@@ -82,6 +82,19 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 #define GB_OOB 0xFFFFFFF0u
 #define GB_FLUSH 8                /* chunks summed in one accumulator (512 values of K) */
 
+/* Waits until at most min(n, N) chunks of LPW loads are out (n < 0: none): a
+ * chunk has landed when only those after it are, of which few follow near K's
+ * end.  (With loads of the last chunk again in their place, so that the count
+ * holds, one chunk of K took seven: 64 x 64, 400 truncated rows 7.2 us, 6.8 now,
+ * 1,328 x 152, 640 rows 8.4 and 8.0.) */
+template <int LPW, int N>
+__device__ __forceinline__ void gb_wait(int n) {
+    if constexpr (N > 0) {
+        if (n < N) return gb_wait<LPW, N - 1>(n);
+    }
+    VMCNT_WAIT(LPW * N);
+}
+
 template <bool HL, int BN>
 __device__ __forceinline__ void gemm_block(const mm_gemm_bf16_args &a, uint8_t *lds) {
     constexpr int NP = HL ? 2 : 1;                 /* A planes: hi (and lo) */
@@ -133,8 +146,8 @@ __device__ __forceinline__ void gemm_block(const mm_gemm_bf16_args &a, uint8_t *
             wk[u] = 8 * ((lane & 7) ^ gb_swz(R));
             wo[u] = R < ncols ? ((uint32_t)R * (uint32_t)K + (uint32_t)wk[u]) * 2u : GB_OOB;
         }
-        auto issue = [&](int kb, int st) {         /* past the last chunk: the last again */
-            const int k0 = min(kb, KB - 1) * GB_BK;
+        auto issue = [&](int kb, int st) {
+            const int k0 = kb * GB_BK;
             const uint32_t sb = lds0 + (uint32_t)(st * SB);
 #pragma unroll
             for (int u = 0; u < 4; u++)
@@ -148,14 +161,18 @@ __device__ __forceinline__ void gemm_block(const mm_gemm_bf16_args &a, uint8_t *
                               sb + (uint32_t)(BOFF + (WL * lw + u) * 1024));
         };
 #pragma unroll 1
-        for (int s = 0; s < NS - 1; s++) issue(s, s);
-        VMCNT_WAIT(LPW * (NS - 2));                /* chunk 0 */
+        for (int s = 0; s < min(NS - 1, KB); s++) issue(s, s);
+        gb_wait<LPW, NS - 2>(KB - 1);              /* chunk 0 */
         __builtin_amdgcn_s_barrier();
-        int st = NS - 1;
-        for (int kb = 0; kb < KB; kb++) {          /* one barrier per chunk */
+        int st = NS - 1, kb = 0;
+        for (; kb + NS - 1 < KB; kb++) {           /* one barrier per chunk */
             issue(kb + NS - 1, st);                /* the slot of chunk kb - 1 */
             st = st + 1 == NS ? 0 : st + 1;
             VMCNT_WAIT(LPW * (NS - 2));            /* chunk kb + 1 */
+            __builtin_amdgcn_s_barrier();
+        }
+        for (; kb < KB; kb++) {
+            gb_wait<LPW, NS - 2>(KB - 2 - kb);
             __builtin_amdgcn_s_barrier();
         }
         VMCNT_WAIT(0);
