@@ -87,12 +87,15 @@ typedef struct {
  * GEMV streams an expert once per token that chose it, the GEMMs once per row
  * tile, but through six launches and at 4-5 TB/s instead of 6.  Up to 64
  * experts only: with more, few tokens share one, and the GEMV stages have the
- * router in their first launch.  Whole layer, GEMV -> GEMM us, for hidden x
+ * router in their first launch; and only with rows of whole 128-byte lines,
+ * which the GEMMs' loads take one line at a time.  Whole layer, GEMV -> GEMM us, for hidden x
  * intermediate size, routed experts, experts per token (+ shared):
  *   2048 x 1408, 64, 6 + 2   5 tokens 120 -> 115, 6: 138 -> 131, 8: 177 -> 154
  *   2048 x 1536, 64, 4 + 1   5 tokens (120 MB saved) 93 -> 95, 6 (159 MB) 106 -> 98
  *   2048 x 1408, 16, 2 + 1   5 tokens (108 MB) 62 -> 63, 6 (141 MB) 69 -> 64
  *   4096 x 14336, 8, 2       5 tokens 648 -> 390
+ *   2176 x 2688, 60, 2 + 2   5 tokens 128 -> 111, 8: 184 -> 133
+ *   2152 x 2712, 60, 2 + 2   5 tokens 132 -> 142, 8: 191 -> 196, 9: 233 -> 199
  *   1024 x 512, 8, 2 + 1     8 tokens (50 MB) 32 -> 35, 9: 50 -> 35
  *   256 x 128, 16, 4 + 2     8 tokens 19 -> 27, 9: 37 -> 27
  *   2048 x 512, 256, 8 + 1   8 tokens 176 -> 211, 9: 277 -> 227 */
