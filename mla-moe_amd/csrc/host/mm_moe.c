@@ -550,7 +550,8 @@ static int bf16_mm_ok(const mm_moe_config *g) {
  * token, each as likely as any other, touch E (1 - (1 - K / E)^T). */
 static int bf16_mm_pays(const mm_moe_config *g, int T) {
     const double E = g->n_routed_experts, K = g->n_experts_per_tok, NS = g->n_shared_experts;
-    if (T > MM_BF16_NT_MAX) return 1;
+    if (T > MM_BF16_NT_MAX)
+        return T > 2 * MM_BF16_NT_MAX || E <= 64 || g->hidden_size >= MM_BF16_MM_TWO_H;
     if (T < MM_BF16_MM_MIN_T || E > 64 || g->hidden_size % 64 || g->moe_inter_size % 64) return 0;
     double untouched = E;
     for (int t = 0; t < T; t++) untouched *= 1 - K / E;

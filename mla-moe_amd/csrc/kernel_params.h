@@ -98,10 +98,20 @@ typedef struct {
  *   2152 x 2712, 60, 2 + 2   5 tokens 132 -> 142, 8: 191 -> 196, 9: 233 -> 199
  *   1024 x 512, 8, 2 + 1     8 tokens (50 MB) 32 -> 35, 9: 50 -> 35
  *   256 x 128, 16, 4 + 2     8 tokens 19 -> 27, 9: 37 -> 27
- *   2048 x 512, 256, 8 + 1   8 tokens 176 -> 211, 9: 277 -> 227 */
+ *   2048 x 512, 256, 8 + 1   8 tokens 176 -> 211, 9: 277 -> 227
+ * Two passes of the GEMV stages (9 to 16 tokens) are still the shorter for more
+ * than 64 experts with a hidden size below MM_BF16_MM_TWO_H: down has few tiles
+ * per expert, too few for the chip:
+ *   208 x 856, 201, 1 + 1    9 tokens 69 -> 76, 16: 75 -> 79, 17: 107 -> 82
+ *   168 x 2832, 106, 2 + 2   9 tokens 75 -> 83
+ *   128 x 128, 256, 8 + 1    9 tokens 77 -> 80
+ *   280 x 2256, 267, 2       9 tokens 75 -> 80
+ *   256 x 256, 128, 1        9 tokens 57 -> 45 (given up by this line)
+ *   512 x 512, 256, 2 + 1    9 tokens 102 -> 98 */
 #ifndef MM_BF16_MM_MIN_T
 #define MM_BF16_MM_MIN_T 5
 #define MM_BF16_MM_SAVED 128e6
+#define MM_BF16_MM_TWO_H 512
 #endif
 #define MM_BF16_NT_MAX 8          /* tokens per pass of the GEMV stages */
 /* Rows of one pass, and bytes of its workspace: 212 KB per row at DeepSeek-V2-Lite's

@@ -73,7 +73,8 @@ def test_shapes(H, E, K, I, NS, T):
     (1024, 4, 2, 2048, 0, 7, 0), (1024, 4, 2, 2048, 0, 8, 1),            # 126 and 151 MB of weights not read again
     (2048, 4, 4, 2048, 0, 4, 0), (2048, 4, 4, 2048, 0, 5, 1),            # 4 tokens stay with the GEMV
     (512, 65, 8, 2048, 4, 8, 0),                                         # more than 64 experts
-    (2048, 4, 4, 2056, 0, 8, 0), (2056, 4, 4, 2048, 0, 8, 0), (2056, 4, 4, 2048, 0, 9, 1)])   # rows of no whole lines
+    (2048, 4, 4, 2056, 0, 8, 0), (2056, 4, 4, 2048, 0, 8, 0), (2056, 4, 4, 2048, 0, 9, 1),    # rows of no whole lines
+    (64, 65, 2, 64, 1, 16, 0), (64, 65, 2, 64, 1, 17, 1), (64, 64, 2, 64, 1, 9, 1), (512, 65, 2, 64, 1, 9, 1)])   # many narrow experts
 def test_rule(H, E, K, I, NS, T, grouped):
     w, x = synth.moe_layer(940, H, E, I, NS), synth.activations(941, T, H)
     with mlamoe.Context(0) as ctx:
